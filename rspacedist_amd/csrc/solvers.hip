@@ -10,6 +10,7 @@
 #include <cstring>
 #include <memory>
 
+#include "gemm_f64.hpp"
 #include "gemm_mixed.hpp"
 #include "kukan_internal.hpp"
 #include "solvers.hpp"
@@ -954,12 +955,14 @@ static void dgemm(rocblas_operation ta, rocblas_operation tb, int m, int n, int 
 }
 
 // C(M x M) = alpha A^T B + beta C in FP64 where the consumer reads one triangle only (tri 1:
-// on and below the diagonal, 2: on and above): the b (b + 1) / 2 blocks of a b x b partition
+// on and below the diagonal, 2: on and above).  Where the matrix-core kernel does not apply, the
+// b (b + 1) / 2 blocks of a b x b partition
 // that hold it, b = param "gram_blocks" (default 4) limited to blocks of at least 256 columns
 // (narrower blocks ran slower than the full product).  At 2,097,152 x 1024 x 1024: 44 ms
 // against 69 ms for the full dgemm.  Entries outside the blocks are left as they are.
 static void dgemm_tn_tri(int M, long K, double alpha, const double *A, long lda, const double *B,
                          long ldb, double beta, double *C, long ldc, int tri) {
+  if (gemm_f64_tn(M, M, K, alpha, A, lda, B, ldb, beta, C, ldc, tri, lib().stream)) return;
   const int nbk = tri ? std::max(1, std::min((int)param("gram_blocks", 4.0), M / 256)) : 1;
   if (nbk <= 1) {
     dgemm(rocblas_operation_transpose, rocblas_operation_none, M, M, (int)K, alpha, A, (int)lda, B,
@@ -1009,6 +1012,7 @@ void subspace_tn(int M1, int M2, long K, double alpha, const double *A, long lda
     dgemm_tn_tri(M1, K, alpha, A, lda, B, ldb, beta, C, ldc, tri);
     return;
   }
+  if (gemm_f64_tn(M1, M2, K, alpha, A, lda, B, ldb, beta, C, ldc, 0, s)) return;
   dgemm(rocblas_operation_transpose, rocblas_operation_none, M1, M2, (int)K, alpha, A, (int)lda, B,
         (int)ldb, beta, C, (int)ldc);
 }
@@ -1025,6 +1029,7 @@ void subspace_nn(long R, int K, int M2, double alpha, const double *X, long ldx,
     return;
   }
   if (colsq) throw Error(1, "subspace_nn: column norms come from the split-precision product only");
+  if (c_upper && gemm_f64_nn_upper(R, K, M2, alpha, X, ldx, C, ldc, beta, Y, ldy, s)) return;
   dgemm(rocblas_operation_none, rocblas_operation_none, (int)R, M2, K, alpha, X, (int)ldx, C,
         (int)ldc, beta, Y, (int)ldy);
 }
@@ -1096,8 +1101,7 @@ static void renormalize(Ctx &c, int M, double *psi, double *spsi, double *rsp, d
 // arithmetic (orthogonalization8f.F90:93-376 with l_inp = 0).
 // fp64: the pass runs in FP64 also when the subspace products are split-precision (the
 // closing orthonormalisation of the band update: the bands it returns are orthonormal to
-// FP64 rounding, not to the split products' ~1e-7).  In FP64, G is one rocBLAS dgemm: at
-// 2,097,152 x 1024 dsyrk took 219 ms against about 62 ms for the full dgemm.
+// FP64 rounding, not to the split products' ~1e-7).
 void cholqr(Ctx &c, int M, double *psi, double *spsi, double *rsp, double *hpsi,
             const double *norms, bool fp64) {
   const long n = c.g.n(), n1 = (long)c.pl.nprjmx * c.pl.num_ppcell;
@@ -1133,20 +1137,31 @@ void cholqr(Ctx &c, int M, double *psi, double *spsi, double *rsp, double *hpsi,
   HIPCK(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c.s));
   sync();
   if (hinfo != 0) throw Error(2, "orthogonalization_r_01 (1): wf has negative norm");
+  // X <- X R^-1: as a triangular matrix-core product with R^-1 where that applies (2097152 x
+  // 1024: 31 ms against 43 for dtrsm, which multiplies in blocks too), else by dtrsm
+  double *Ri = nullptr;
+  auto inverse = [&]() {  // R^-1 in FP64 (upper triangular)
+    if (Ri) return;
+    Ri = c.buf("cholqr.Ri", (size_t)M * M);
+    HIPCK(hipMemcpy2DAsync(Ri, sizeof(double) * M, G, sizeof(double) * M, sizeof(double) * M, M,
+                           hipMemcpyDeviceToDevice, c.s));
+    Timed t("trtri", (double)M * M * M / 3.0);
+    BLASCK(rocsolver_dtrtri(h, rocblas_fill_upper, rocblas_diagonal_non_unit, M, Ri, M, info));
+  };
   auto tr = [&](double *X, long ldx, long rows) {
+    if (rows == n && apply_upper_ok(rows, M, X, ldx)) {
+      inverse();
+      Timed t("trsm_f64", (double)rows * M * M);
+      gemm_f64_apply_upper(rows, M, X, ldx, Ri, M, c.s);
+      return;
+    }
     Timed t("trsm_f64", (double)rows * M * M);
     BLASCK(rocblas_dtrsm(h, rocblas_side_right, rocblas_fill_upper, rocblas_operation_none,
                          rocblas_diagonal_non_unit, (int)rows, M, &one, G, M, X, (int)ldx));
   };
   if (split) {
     // R^-1 in FP64 (upper triangular), then X <- X R^-1 as a split-FP16 product
-    double *Ri = c.buf("cholqr.Ri", (size_t)M * M);
-    HIPCK(hipMemcpy2DAsync(Ri, sizeof(double) * M, G, sizeof(double) * M, sizeof(double) * M, M,
-                           hipMemcpyDeviceToDevice, c.s));
-    {
-      Timed t("trtri", (double)M * M * M / 3.0);
-      BLASCK(rocsolver_dtrtri(h, rocblas_fill_upper, rocblas_diagonal_non_unit, M, Ri, M, info));
-    }
+    inverse();
     hipLaunchKernelGGL(k_zero_lower, dim3(nblk((long)M * M, 256)), dim3(256), 0, c.s, M, Ri);
     // in place: the split product reads X only through its pre-split copy
     auto apply = [&](double *X, const double *sx, const SplitBands *px) {

@@ -1,0 +1,76 @@
+"""The FP64 matrix-core products at the edges of their tiles, against numpy in extended precision.
+
+Bound: a sum of K products in any order is off by at most K 2^-53 (1 + O(K 2^-53)) times the sum
+of their absolute values (numpy's longdouble reference adds nothing at this level)."""
+import numpy as np
+import pytest
+
+from rspacedist_amd import synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def kk():
+    from rspacedist_amd import kukan
+    kukan.init(0)
+    kukan.set_param("precision", 0)
+    return kukan
+
+
+# one column .. past a tile of 64 and 128 on either side; inner lengths below, at and past a
+# 16-deep step, and odd ones (columns that are not 16-byte aligned)
+@pytest.mark.parametrize("m1,m2,k", [(1, 1, 1), (3, 5, 15), (16, 16, 16), (64, 64, 17), (65, 63, 257), (128, 128, 4096),
+                                     (129, 127, 4098), (130, 130, 4097), (200, 131, 1000), (300, 70, 2049),
+                                     (70, 300, 333), (260, 260, 515)])
+@pytest.mark.parametrize("beta", [0.0, -0.5])
+def test_tn_product(kk, m1, m2, k, beta):
+    rng = np.random.default_rng(m1 * 1000 + m2 + k)
+    A, B = (np.asfortranarray(rng.standard_normal((k, m))) for m in (m1, m2))
+    C0 = np.asfortranarray(rng.standard_normal((m1, m2)))
+    C = C0.copy(order="F") if beta else np.full_like(C0, np.nan)  # beta = 0 must not read C
+    kk.subspace_gemm(1, m1, m2, k, 0.7, A, k, B, k, beta, C, m1)
+    ref = 0.7 * (A.astype(np.longdouble).T @ B.astype(np.longdouble)) + beta * C0
+    bound = (k + 4) * 2.0 ** -53 * (0.7 * (np.abs(A).T @ np.abs(B)) + np.abs(beta * C0))
+    assert np.all(np.abs(C - ref) <= bound)
+
+
+@pytest.mark.parametrize("n,m", [(12, 5), (11, 70), (12, 129), (16, 300)])
+def test_orthogonalisation_triangles(kk, n, m):
+    """orthogonalization_r forms a Gram triangle and applies the triangular inverse in place, over
+    one to three column tiles and for even and odd band lengths: Q^T Q dV = 1, and Q spans the
+    input with the positive-diagonal factor of the Householder QR.  Random bands have a Gram
+    condition number kappa of order 10, and both factorisations are off by a few n eps kappa."""
+    s = synth.make_system(n, 0.4, 2, m, seed=n + m)
+    psi0 = synth.random_bands(s)
+    psi = psi0.copy(order="F")
+    kk.call("orthogonalization_r", **synth.abi_args(s), nflag=1, svecre=psi, ssvre=psi,
+            rspsep=np.zeros((9, s.natom, m), order="F"))
+    kappa = np.linalg.cond(psi0) ** 2
+    np.testing.assert_allclose(psi.T @ psi * s.dv, np.eye(m), rtol=0, atol=s.npts * 2.0 ** -53 * kappa)
+    q, r = np.linalg.qr(psi0 * np.sqrt(s.dv))
+    q *= np.sign(np.diag(r))
+    np.testing.assert_allclose(psi * np.sqrt(s.dv), q, rtol=0, atol=s.npts * 2.0 ** -53 * kappa)
+
+
+@pytest.mark.parametrize("m", [66, 130, 257])
+def test_block_cg_projection_triangle(kk, m):
+    """One block-CG step in FP64 with the triangular projection product and with every product
+    on rocBLAS (params gemm_f64 1 / 0): the same step to rounding."""
+    s = synth.make_system(14, 0.35, 2, m, seed=m)
+    psi = synth.smooth_bands(synth.random_bands(s), s.n, s.h, width=0.6 * s.h)
+    out = []
+    for own in (1, 0):
+        kk.set_param("gemm_f64", own)
+        kk.set_param("kscg_mode", 1)
+        st = dict(svecre=psi.copy(order="F"), rspsep=np.zeros((9, s.natom, m), order="F"), sval=np.zeros(m),
+                  residual_states=np.zeros(m), hsvre=np.zeros_like(psi, order="F"))
+        st["ssvre"] = st["svecre"]
+        kk.call("orthogonalization_r", **synth.abi_args(s), nflag=1, **{k: st[k] for k in ("svecre", "ssvre", "rspsep")})
+        kk.call("scf_diag", **synth.abi_args(s, nsdmax=2, epssd=1e-14), **st)
+        out.append(st)
+        kk.set_param("gemm_f64", 1)
+        kk.set_param("kscg_mode", 0)
+    np.testing.assert_allclose(out[0]["sval"], out[1]["sval"], rtol=0, atol=1e-10 * np.abs(out[1]["sval"]).max())
+    rho = [(o["svecre"] ** 2).sum(axis=1) for o in out]
+    np.testing.assert_allclose(rho[0], rho[1], rtol=0, atol=1e-9 * rho[1].max())
