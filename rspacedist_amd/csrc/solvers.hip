@@ -12,6 +12,7 @@
 
 #include "gemm_f64.hpp"
 #include "gemm_mixed.hpp"
+#include "hartree_cg.hpp"
 #include "kukan_internal.hpp"
 #include "solvers.hpp"
 
@@ -457,73 +458,12 @@ __global__ void k_sub_scalar(long n, const double *s, double f, double *x) {
   const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
   if (i < n) x[i] = x[i] - s[0] * f;
 }
-// Hartree CG updates (scf_hartree8f.F90:849-891); scalars on the device: sc[0]=r1r, sc[1]=pap
-// Device-side Hartree CG loop state: st[0] = done, st[1] = current iteration (1-based).
-// Every kernel of an iteration returns at once when done is set, so a block of iterations
-// can be launched (or replayed as a graph) past convergence without changing the result.
-// An iteration is four launches: A p (stencil, with <p|A p> partials), the update (each
-// work-group folds the stencil partials itself), the direction (each work-group folds the
-// update's <r|r> partials itself) and the stopping rule of scf_hartree8f.F90.
+// state of the device-side CG loop (hartree_cg.hpp): not done, at iteration 1
 __global__ void k_hcg_reset(int *st) {
   st[0] = 0;
   st[1] = 1;
+  st[2] = 0;
 }
-// Sum of np partials by a 256-thread work-group in a fixed order (strided per thread, then
-// wave shuffles, then the 4 wave sums in order); every thread gets the result.
-__device__ inline double fold_parts256(const double *part, int np, double *red4) {
-  double s = 0.0;
-  for (int c = threadIdx.x; c < np; c += 256) s += part[c];
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if ((threadIdx.x & 63) == 0) red4[threadIdx.x >> 6] = s;
-  __syncthreads();
-  const double tot = ((red4[0] + red4[1]) + red4[2]) + red4[3];
-  __syncthreads();
-  return tot;
-}
-__global__ void k_hcg_update(long n, const double *sc, double *vh, const double *p, const double *ap,
-                             double *avhs, const double *b, double *r, const double *spart,
-                             int nsp, double *part, int nparts, const int *st) {
-  __shared__ double red[4];
-  if (st[0]) return;
-  const double alph = sc[0] / fold_parts256(spart, nsp, red);  // r1r / pap
-  const long chunk = (n + nparts - 1) / nparts;
-  const long i0 = blockIdx.x * chunk, i1 = min(n, i0 + chunk);
-  double s = 0.0;
-  for (long i = i0 + threadIdx.x; i < i1; i += 256) {
-    vh[i] = vh[i] + alph * p[i];
-    avhs[i] = avhs[i] + alph * ap[i];
-    const double ri = b[i] - avhs[i];
-    r[i] = ri;
-    s += ri * ri;
-  }
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) part[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
-}
-__global__ void k_hcg_dir(long n, double *sc, const double *upart, int nup, int ncgres,
-                          const double *r, double *p, const int *st) {
-  __shared__ double red[4];
-  if (st[0]) return;
-  const double r2r = fold_parts256(upart, nup, red);
-  const double beta = (st[1] % ncgres == 0) ? 0.0 : r2r / sc[0];
-  if (blockIdx.x == 0 && threadIdx.x == 0) sc[2] = r2r;
-  const long stride = (long)gridDim.x * 256;
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < n; i += stride) p[i] = r[i] + beta * p[i];
-}
-// stopping rule (ncgmin, ncgmax, dp = sqrt(r.r dV / Omega) <= epsvh); else next iteration
-__global__ void k_hcg_ctl(double *sc, double dvo, double eps, int ncgmin, int ncgmax, int *st) {
-  if (st[0]) return;
-  const int loop = st[1];
-  const double dp = sqrt(sc[2] * dvo);
-  if (loop >= ncgmin && (loop >= ncgmax || dp <= eps)) {
-    st[0] = 1;
-    return;
-  }
-  st[1] = loop + 1;
-  sc[0] = sc[2];
-}
-
 
 // ---------------------------------------------------------------- persistent Hartree CG
 // The whole CG loop of scf_hartree8f.F90:611-1143 in one cooperative launch (opt-in, param
@@ -1773,16 +1713,17 @@ void reorder(Ctx &c, int M, double *sval, double *resid, double *psi, double *sp
 // ============================================================================= Hartree
 // scf_hartree8f.F90:11-812: b = 2 pi rho (+ Dirichlet planes), periodic mean removed, CG on
 // -1/2 lap_nfh with the reference's avhs recurrence and stopping rule.
-// Layout of one solve's buffers: b, r, p, ap, avhs (n each), then sc (16), the stencil /
-// update partials (max(np, npu)), the update partials (npu), the dot partials
-// (dot_nparts(n)), the boundary weights (3 x 9) and the state (2 ints), each 256-byte aligned.
+// Layout of one solve's buffers: b, r, two directions (the second also the persistent CG's
+// avhs) and A p (n each), then sc (16), the partials of the two kernels (HCG_PARTS each), the dot
+// partials (dot_nparts(n)), the boundary weights (3 x 9) and the state (3 ints), each 256-byte
+// aligned.
 namespace {
 struct HartreeBufs {
-  double *b, *r, *p, *ap, *avhs, *sc, *part, *upart, *dpart, *w;
+  double *b, *r, *p, *p2, *ap, *sc, *part, *upart, *dpart, *w;
   int *state;
   size_t bytes;
 };
-HartreeBufs hartree_layout(char *base, long n, int np, int npu) {
+HartreeBufs hartree_layout(char *base, long n) {
   HartreeBufs o{};
   size_t off = 0;
   auto take = [&](size_t bytes) {
@@ -1793,27 +1734,18 @@ HartreeBufs hartree_layout(char *base, long n, int np, int npu) {
   o.b = (double *)take(sizeof(double) * n);
   o.r = (double *)take(sizeof(double) * n);
   o.p = (double *)take(sizeof(double) * n);
+  o.p2 = (double *)take(sizeof(double) * n);
   o.ap = (double *)take(sizeof(double) * n);
-  o.avhs = (double *)take(sizeof(double) * n);
   o.sc = (double *)take(sizeof(double) * 16);
-  o.part = (double *)take(sizeof(double) * std::max(np, npu));
-  o.upart = (double *)take(sizeof(double) * npu);
+  o.part = (double *)take(sizeof(double) * HCG_PARTS);
+  o.upart = (double *)take(sizeof(double) * HCG_PARTS);
   o.dpart = (double *)take(sizeof(double) * dot_nparts(n));
   o.w = (double *)take(sizeof(double) * 27);
-  o.state = (int *)take(sizeof(int) * 2);
+  o.state = (int *)take(sizeof(int) * 3);
   o.bytes = off;
   return o;
 }
-int hartree_update_parts(long n) {
-  const long chunk = (long)param("hart_upd_chunk", 4096.0);
-  return (int)std::min<long>(1024, std::max<long>(1, (n + chunk - 1) / chunk));
-}
 }  // namespace
-
-size_t hartree_work_bytes(const Grid &g, int nfh) {
-  const long n = g.n();
-  return hartree_layout(nullptr, n, stencil_nparts(g, nfh, 1), hartree_update_parts(n)).bytes;
-}
 
 // The persistent CG (k_hcg_persistent) when the grid fits one cooperative launch of resident
 // work-groups: returns the iterations, or 0 when it does not apply (the caller then runs the
@@ -1882,28 +1814,14 @@ int hartree(const HartreeArgs &a, const HartreeWork *ws) {
          2.0 * a.zmax / a.nz};
   const long n = g.n();
   const double omega = 8.0 * a.xmax * a.ymax * a.zmax;
-  const int np = stencil_nparts(g, a.nfh, 1);
-  // update work-groups: 4096 points each (512 at 128^3; 8192 points each, one work-group per
-  // CU, left the update latency-bound: a 128^3 solve took 33.9 ms against 29.7)
-  const int npu = hartree_update_parts(n);
   HartreeBufs B;
   if (ws) {
-    B = hartree_layout(ws->base, n, np, npu);
+    B = hartree_layout(ws->base, n);
     if (B.bytes > ws->bytes) throw Error(1, "scf_hartree: workspace too small for this grid");
   } else {
-    B.b = (double *)scratch("hart.b", sizeof(double) * n);
-    B.r = (double *)scratch("hart.r", sizeof(double) * n);
-    B.p = (double *)scratch("hart.p", sizeof(double) * n);
-    B.ap = (double *)scratch("hart.ap", sizeof(double) * n);
-    B.avhs = (double *)scratch("hart.avhs", sizeof(double) * n);
-    B.sc = (double *)scratch("hart.sc", sizeof(double) * 16);
-    B.part = (double *)scratch("hart.part", sizeof(double) * std::max(np, npu));
-    B.upart = (double *)scratch("hart.upart", sizeof(double) * npu);
-    B.dpart = nullptr;  // launch_dots' own buffer
-    B.w = (double *)scratch("hart.w", sizeof(double) * 27);
-    B.state = (int *)scratch("hart.state", sizeof(int) * 2);
+    B = hartree_layout((char *)scratch("hart.work", hartree_layout(nullptr, n).bytes), n);
   }
-  double *b = B.b, *r = B.r, *p = B.p, *ap = B.ap, *avhs = B.avhs, *sc = B.sc, *part = B.part;
+  double *b = B.b, *r = B.r, *p = B.p, *ap = B.ap, *sc = B.sc;
   hipLaunchKernelGGL(k_hartree_b, dim3(nblk(n, 256)), dim3(256), 0, s, n, a.rho, b);
   double w[9];
   fd_coefficients(a.nfh, w);
@@ -1935,40 +1853,45 @@ int hartree(const HartreeArgs &a, const HartreeWork *ws) {
   st.g = &g; st.in = a.vh; st.ld_in = n; st.out = ap; st.ld_out = n; st.veff = nullptr;
   st.nb = 1; st.nfh_coeffs = a.nfh;
   launch_stencil(st, s);
-  HIPCK(hipMemcpyAsync(avhs, ap, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
   launch_axpby(n, 1, nullptr, 1.0, b, n, nullptr, -1.0, ap, n, r, n, s);
-  HIPCK(hipMemcpyAsync(p, r, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
-  // CG iterations run as blocks of `blk` on the device (scf_hartree8f.F90:611-1143): the
-  // stopping rule is evaluated on the device after every iteration and later iterations of
-  // the block do nothing, so the result is that of the host-driven loop; the host reads the
-  // state once per block.  With param "hartree_graph" (default 1) a block is captured once
-  // as a HIP graph and replayed.
   int *state = B.state;
-  double *upart = B.upart;
-  hipLaunchKernelGGL(k_hcg_reset, dim3(1), dim3(1), 0, s, state);
-  launch_dots(n, r, n, r, n, 1, 1.0, sc + 0, s, B.dpart);  // r1r of iteration 1
-  st.in = p; st.out = ap; st.dot_partial = part; st.skip = state;
   const double dvo = g.dv() / omega;
   lib().params["hartree_persistent_used"] = 0.0;
-  // opt-in: at 128^3 it takes 47 us per iteration against 55 for the iteration blocks, at
-  // 96^3 and 64^3 45 / 38 against 43 / 34 (its iterations are bound by memory round trips)
+  // opt-in: one cooperative launch (47 us per iteration at 128^3, 45 / 38 at 96^3 / 64^3)
   if (!ws && param("hartree_persistent", 0.0) >= 1.0) {
-    const int loops = hartree_persistent(a, g, n, b, p, avhs, sc, dvo, state);
+    HIPCK(hipMemcpyAsync(B.p2, ap, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
+    HIPCK(hipMemcpyAsync(p, r, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
+    launch_dots(n, r, n, r, n, 1, 1.0, sc, s, B.dpart);
+    const int loops = hartree_persistent(a, g, n, b, p, B.p2, sc, dvo, state);
     if (loops > 0) {
       lib().params["hartree_persistent_used"] = 1.0;
       return loops;
     }
   }
-  const int blk = std::max(1, (int)param("hartree_block", 16.0));
-  auto iteration = [&]() {
-    launch_stencil(st, s);
-    hipLaunchKernelGGL(k_hcg_update, dim3(npu), dim3(256), 0, s, n, sc, a.vh, p, ap, avhs, b, r,
-                       part, np, upart, npu, state);
-    hipLaunchKernelGGL(k_hcg_dir, dim3(std::min(nblk(n, 256), 2048u)), dim3(256), 0, s, n, sc, upart, npu,
-                       a.ncgres, r, p, state);
-    hipLaunchKernelGGL(k_hcg_ctl, dim3(1), dim3(1), 0, s, sc, dvo, a.epsvh, a.ncgmin, a.ncgmax,
-                       state);
-  };
+  // CG iterations run as blocks of `blk` on the device (scf_hartree8f.F90:611-1143): the
+  // stopping rule is evaluated on the device and the later iterations of a block do nothing, so
+  // the result is that of the host-driven loop; the host reads the state once per block.  With
+  // param "hartree_graph" (default 1) a block is captured once as a HIP graph and replayed.
+  HcgArgs cg{};
+  cg.nx = a.nx; cg.ny = a.ny; cg.nz = a.nz;
+  cg.px = a.nperi >= 1; cg.py = a.nperi >= 2; cg.pz = a.nperi >= 3;
+  for (int m = 0; m <= a.nfh; m++) {
+    cg.cx[m] = w[m] / g.dx / g.dx * (-0.5);
+    cg.cy[m] = w[m] / g.dy / g.dy * (-0.5);
+    cg.cz[m] = w[m] / g.dz / g.dz * (-0.5);
+  }
+  cg.c0 = cg.cx[0] + cg.cy[0] + cg.cz[0];
+  cg.n = n; cg.vh = a.vh; cg.r = r; cg.p[0] = p; cg.p[1] = B.p2; cg.ap = ap;
+  cg.part_p = B.part; cg.part_r = B.upart; cg.rr = sc; cg.state = state;
+  cg.ncgres = a.ncgres; cg.ncgmin = a.ncgmin; cg.ncgmax = a.ncgmax; cg.dvo = dvo; cg.eps = a.epsvh;
+  hcg_plan(cg, a.nfh);
+  hipLaunchKernelGGL(k_hcg_reset, dim3(1), dim3(1), 0, s, state);
+  launch_fill(n, 0.0, p, s);                               // iteration 1 takes beta = 0
+  launch_dots(n, r, n, r, n, 1, 1.0, sc + 1, s, B.dpart);  // <r|r> before iteration 1
+  // an even number of iterations per block: the direction alternates between two buffers.  32: a
+  // block past convergence costs less than another host read (40^3: 1.87 ms against 1.98 with 16)
+  const int blk = std::max(2, ((int)param("hartree_block", 32.0) + 1) / 2 * 2);
+  auto iteration = [&](int it) { hcg_iteration(cg, a.nfh, it & 1, s); };
   // a captured block is valid for the same buffers, sizes and stopping parameters
   struct Key {
     std::vector<const void *> ptrs;
@@ -1985,8 +1908,8 @@ int hartree(const HartreeArgs &a, const HartreeWork *ws) {
   static GraphCache gc;
   const bool use_graph = !ws && param("hartree_graph", 1.0) >= 1.0;
   if (use_graph) {
-    const Key key{{a.vh, b, r, p, ap, avhs, sc, part, upart, state},
-                  {n, a.nx, a.ny, a.nz, a.nperi, a.nfh, blk, a.ncgres, a.ncgmin, a.ncgmax, np, npu},
+    const Key key{{a.vh, r, p, B.p2, ap, sc, B.part, B.upart, state},
+                  {n, a.nx, a.ny, a.nz, a.nperi, a.nfh, blk, a.ncgres, a.ncgmin, a.ncgmax, cg.tx, cg.tz},
                   {a.epsvh, dvo, g.dx, g.dy, g.dz}};
     if (!(gc.exec && gc.key == key)) {
       if (gc.exec) HIPCK(hipGraphExecDestroy(gc.exec));
@@ -1995,7 +1918,7 @@ int hartree(const HartreeArgs &a, const HartreeWork *ws) {
       lib().capturing = true;
       try {
         HIPCK(hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed));
-        for (int it = 0; it < blk; it++) iteration();
+        for (int it = 0; it < blk; it++) iteration(it);
         HIPCK(hipStreamEndCapture(s, &graph));
       } catch (...) {
         lib().capturing = false;
@@ -2009,17 +1932,17 @@ int hartree(const HartreeArgs &a, const HartreeWork *ws) {
       gc.key = key;
     }
   }
-  int hst[2] = {0, 0};
+  int hst[3] = {0, 0, 0};
   for (;;) {
     if (use_graph) HIPCK(hipGraphLaunch(gc.exec, s));
     else
-      for (int it = 0; it < blk; it++) iteration();
+      for (int it = 0; it < blk; it++) iteration(it);
     HIPCK(hipMemcpyAsync(hst, state, sizeof(hst), hipMemcpyDeviceToHost, s));
     sync();
-    if (hst[0]) break;
-    if (hst[1] > a.ncgmax) break;  // not reached: the stopping rule sets done at ncgmax
+    if (hst[0]) return hst[2];
+    // not reached: the rule after iteration max(ncgmin, ncgmax) sets done in the next one
+    if (hst[1] > std::max(a.ncgmin, a.ncgmax) + 2 * blk) return hst[1] - 1;
   }
-  return hst[1];
 }
 
 void correct_potential(long n, double dvol_over_omega, double *vh) {

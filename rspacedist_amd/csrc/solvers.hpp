@@ -107,14 +107,11 @@ void ksdiis(Ctx &c, const DiisArgs &a);
 void reorder(Ctx &c, int M, double *sval, double *resid, double *psi, double *spsi, double *rsp,
              double *hpsi, bool move_h = false, bool h_scratch = false);
 // Buffers of one Hartree solve carved from a caller's workspace instead of the library's
-// own allocations: 5 grid vectors and the small arrays (see hartree_work_bytes).
+// own allocations: 5 grid vectors and the small arrays.
 struct HartreeWork {
   char *base;
   size_t bytes;
 };
-// bytes a Hartree solve on a grid of n points needs in a HartreeWork (0 if the grid's
-// partial-sum counts are unknown before set-up: never for the tiled stencil)
-size_t hartree_work_bytes(const Grid &g, int nfh);
 // ws: run on the caller's workspace with eager launches (no graph, no allocation)
 int hartree(const HartreeArgs &a, const HartreeWork *ws = nullptr);
 void correct_potential(long n, double dvol_over_omega, double *vh);

@@ -1,0 +1,58 @@
+"""The Hartree CG's tiled iteration on grids whose edges do not fill its tiles (32 x 8 or 16 x 16
+columns; 2, 4 or 8 planes), every stencil width and number of periodic directions, against the
+solution by the eigenvectors of each axis' operator.
+
+Bar: the solve stops at sqrt(mean r^2) <= eps, so |V - V*| <= eps sqrt(n) / lambda_min with
+lambda_min the operator's smallest nonzero eigenvalue."""
+import numpy as np
+import pytest
+
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def kk():
+    from rspacedist_amd import kukan
+    kukan.init(0)
+    kukan.set_param("hartree_persistent", 0)
+    return kukan
+
+
+def _axis(n, h, nf, periodic):
+    a = -0.5 * H.fd_weights(nf) / h ** 2
+    t = np.zeros((n, n))
+    for i in range(n):
+        t[i, i] += a[0]
+        for m in range(1, nf + 1):
+            for j in (i - m, i + m):
+                if periodic or 0 <= j < n:
+                    t[i, j % n] += a[m]
+    return np.linalg.eigh(t)
+
+
+@pytest.mark.parametrize("dims", [(8, 8, 8), (33, 9, 13), (16, 17, 6), (47, 31, 34), (64, 40, 100), (70, 66, 68),
+                                  (258, 10, 9)])
+@pytest.mark.parametrize("nperi,nfh", [(3, 4), (0, 6), (1, 5), (2, 4)])
+def test_tiles(kk, dims, nperi, nfh):
+    h, eps = 0.3, 1e-9
+    if min(dims) < nfh:
+        pytest.skip("edge below the stencil radius")
+    rng = np.random.default_rng(sum(dims) + nperi)
+    rho = np.asfortranarray(rng.random(dims))
+    v = np.asfortranarray(0.1 * rng.standard_normal(dims))  # a warm start far from the solution
+    z = np.zeros(1)
+    kk.call("scf_hartree", nd=1, ncpx_d=dims[0], ncpy_d=dims[1], ncpz_d=dims[2], nfh=nfh, ndisp=6, nperi=nperi,
+            ncgres=801, ncgmin=1, ncgmax=3000, xmax=dims[0] * h / 2, ymax=dims[1] * h / 2, zmax=dims[2] * h / 2,
+            epsvh=eps, rho_aug_dense=rho, boundx=z, boundy=z, boundz=z, vh_dense=v)
+    b = 2 * np.pi * rho
+    if nperi == 3:
+        b, v = b - b.mean(), v - v.mean()
+    lam, q = zip(*(_axis(n, h, nfh, nperi > ax) for ax, n in enumerate(dims)))
+    c = np.einsum("xyz,xa,yb,zc->abc", b, *q, optimize=True)
+    d = lam[0][:, None, None] + lam[1][None, :, None] + lam[2][None, None, :]
+    live = d > 1e-8
+    ref = np.einsum("abc,xa,yb,zc->xyz", np.where(live, c / np.where(live, d, 1.0), 0.0), *q, optimize=True)
+    assert np.linalg.norm(v - ref) <= 1.01 * eps * np.sqrt(rho.size) / d[live].min()
+    assert kk.get_param("hartree_iterations") < 3000
