@@ -692,12 +692,13 @@ int kukan_scf_charge_smt_r(int neigmx, int nums, int nspv, int numk, int ncpx, i
   Arr F(fnele, (size_t)nall * D, Arr::In);
   Arr Ps(svecre, (size_t)n * nall * D, Arr::In);
   Arr Rho(rhosmt, (size_t)n * nspv * D, Arr::Out);
-  launch_fill(n * nspv, 0.0, Rho.d(), lib().stream);
+  // channels without a spin of their own stay zero; the others start with their first contribution
+  if (nspv > nums) launch_fill(n * (nspv - nums), 0.0, Rho.d() + (size_t)n * nums, lib().stream);
   for (int ns = 1; ns <= nums; ns++) {
     const int nsr = std::min(ns, nspv);
     for (int nk = 1; nk <= numk; nk++) {
       const size_t b = (size_t)neigmx * ((ns - 1) + (size_t)nums * (nk - 1));
-      charge(n, neigmx, Ps.d() + n * b, F.d() + b, Rho.d() + (size_t)n * (nsr - 1));
+      charge(n, neigmx, Ps.d() + n * b, F.d() + b, Rho.d() + (size_t)n * (nsr - 1), nk > 1 || nsr < ns);
     }
   }
   Rho.finish();

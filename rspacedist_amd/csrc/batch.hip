@@ -580,8 +580,7 @@ void hartree_start(Batch &B, int s0, int s1, bool batched, hipStream_t s) {
   const int ns = s1 - s0;
   for (int i = s0; i < s1; i++) {
     BatchSystem &S = *B.sys[i];
-    launch_fill(S.g.n(), 0.0, S.rho, s);
-    charge(S.g.n(), S.M, S.psi, S.ones, S.rho);
+    charge(S.g.n(), S.M, S.psi, S.ones, S.rho, false);
   }
   HSys *hs = B.hs + s0;
   double *part = B.hpart + (long)s0 * HCH;

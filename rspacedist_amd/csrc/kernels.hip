@@ -161,6 +161,7 @@ __global__ __launch_bounds__(256) void k_stencil(SP p) {
 //     combination is never stored and the stencil loads only x; it also sums <y|out>.
 //     MODE 5 is MODE 2 without y: for a symmetric H, <y|H p> = ca_b <H y|x> + cb_b <y|H y>,
 //     so the block sums <ca_b x|out> and <ca_b x|H y> from x and H y alone and y is not read.
+//   * MODE 7 is the plain form without the store: only the partials of <c|out>.
 //   * MODE 6 (radius 1) is the block CG's band update fused with the next residual
 //     preconditioner: every value it loads is formed as xn = ca_b x + cb_b y (the new band),
 //     un = ha_b h + hb_b w (its H) and r = sign (un - eps_b xn); out = K r, and the centre's
@@ -387,7 +388,7 @@ __device__ inline void stencil_block(const SL &p, int b, int tile, int zch, doub
       }
       if (!NORMS && p.omax) amax = fmax(amax, fabs(s));
       const long r = zh + oxy[q];
-      out[r] = p.accumulate ? out[r] + s : s;
+      if (MODE != 7) out[r] = p.accumulate ? out[r] + s : s;
       if (UPD) {
         p.out_x[(long)b * p.ld_out + r] = xcen[q];
         p.out_h[(long)b * p.ld_out + r] = ucen[q];
@@ -608,6 +609,111 @@ __global__ __launch_bounds__(256) void k_gather(const int *act, int num_list, in
       double *o = rp + (long)(b0 + q) * ld_rp + j + (long)nprjmx * slot;
       *o = accumulate ? *o + s : s;
     }
+  }
+}
+
+// The same contraction on the matrix cores for 16 bands: rows = the projectors of T tables on
+// one list (vnlocp alone, or with its three derivatives), columns = bands, inner dimension = the
+// atom's list points.  Lane l holds, for a step of 16 points, the four points 4 (l / 16) .. + 3:
+// of table row l % 16 as 32 consecutive bytes, of band l % 16 as four gathered values (MFMA s of
+// the step takes value s on both sides).  A table value is read once per 16 bands instead of once
+// per 4, and psi's list points once for all tables.  The four waves take the steps in turn and
+// their sums are added in wave order.
+typedef double gd4 __attribute__((ext_vector_type(4)));
+typedef double gd4u __attribute__((ext_vector_type(4), aligned(8)));
+typedef int gi4u __attribute__((ext_vector_type(4), aligned(4)));
+struct GatherArgs {
+  const int *act, *lst;
+  int num_list, nprjmx, nb, ntab, accumulate;
+  const double *tab[4], *psi;
+  long ld;
+  double *out[4];  // per table: (nprjmx num_ppcell) per band
+  long ld_out;
+};
+template <int RT>
+__global__ __launch_bounds__(256) void k_gather_mfma(GatherArgs g) {
+  __shared__ double red[4][16 * RT * 16];
+  const int a = blockIdx.y, t = threadIdx.x, lane = t & 63, w = t >> 6, q = lane >> 4, c16 = lane & 15;
+  const int slot = g.act[5 * a], natinf = g.act[5 * a + 1], iprj = g.act[5 * a + 2];
+  const int b0 = blockIdx.x * 16, nrow = g.ntab * iprj;
+  const double *v = g.psi + g.ld * min(b0 + c16, g.nb - 1);  // bands past the end: results unused
+  const int *ls = g.lst + (long)g.num_list * slot;
+  const double *pt[RT];
+#pragma unroll
+  for (int r = 0; r < RT; r++) {
+    const int row = min(16 * r + c16, nrow - 1), d = row / iprj, j = row - d * iprj;
+    const double *base = d == 0 ? g.tab[0] : d == 1 ? g.tab[1] : d == 2 ? g.tab[2] : g.tab[3];
+    pt[r] = base + (long)g.num_list * ((long)g.nprjmx * slot + j);
+  }
+  gd4 acc[RT];
+#pragma unroll
+  for (int r = 0; r < RT; r++) acc[r] = gd4{0.0, 0.0, 0.0, 0.0};
+  const int full = natinf / 16;
+  // one row tile: a step's list entries are loaded two steps ahead and its values one step ahead;
+  // more row tiles have enough waves' worth of loads per step, and fewer registers to spare
+  auto entries = [&](int st) { return *(const gi4u *)(ls + 16 * min(st, full - 1) + 4 * q); };
+  auto values = [&](int st, gi4u i4, gd4u (&x)[RT], double (&y)[4]) {
+    const int k = 16 * min(st, full - 1) + 4 * q;
+#pragma unroll
+    for (int s = 0; s < 4; s++) y[s] = v[i4[s] - 1];
+#pragma unroll
+    for (int r = 0; r < RT; r++) x[r] = *(const gd4u *)(pt[r] + k);
+  };
+  if constexpr (RT > 1) {
+    for (int st = w; st < full; st += 4) {
+      gd4u x[RT];
+      double y[4];
+      values(st, entries(st), x, y);
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+#pragma unroll
+        for (int r = 0; r < RT; r++) acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[r][s], y[s], acc[r], 0, 0, 0);
+    }
+  } else if (w < full) {
+    gd4u x[2][RT];
+    double y[2][4];
+    gi4u in = entries(w);
+    values(w, in, x[0], y[0]);
+    in = entries(w + 4);
+    for (int st = w; st < full; st += 8) {
+#pragma unroll
+      for (int u = 0; u < 2; u++) {
+        if (st + 4 * u >= full) break;
+        const gi4u nx = entries(st + 4 * u + 8);
+        values(st + 4 * u + 4, in, x[1 - u], y[1 - u]);
+        in = nx;
+#pragma unroll
+        for (int s = 0; s < 4; s++)
+#pragma unroll
+          for (int r = 0; r < RT; r++)
+            acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[u][r][s], y[u][s], acc[r], 0, 0, 0);
+      }
+    }
+  }
+  if (16 * full < natinf && w == (full & 3)) {  // the last, partial step: zeros past natinf on both sides
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      const int k = 16 * full + 4 * q + s;
+      const bool in = k < natinf;
+      const double y = in ? v[ls[k] - 1] : 0.0;
+#pragma unroll
+      for (int r = 0; r < RT; r++)
+        acc[r] = __builtin_amdgcn_mfma_f64_16x16x4f64(in ? pt[r][k] : 0.0, y, acc[r], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < RT; r++)
+#pragma unroll
+    for (int e = 0; e < 4; e++) red[w][(16 * r + q + 4 * e) * 16 + c16] = acc[r][e];
+  __syncthreads();
+  for (int e = t; e < nrow * 16; e += 256) {  // consecutive threads: the rows of one band
+    const int row = e % nrow, c = e / nrow, i = row * 16 + c;
+    if (b0 + c >= g.nb) continue;
+    const double s = ((red[0][i] + red[1][i]) + red[2][i]) + red[3][i];
+    const int d = row / iprj, j = row - d * iprj;
+    double *base = d == 0 ? g.out[0] : d == 1 ? g.out[1] : d == 2 ? g.out[2] : g.out[3];
+    double *o = base + g.ld_out * (b0 + c) + (long)g.nprjmx * slot + j;
+    *o = g.accumulate ? *o + s : s;
   }
 }
 
@@ -1166,6 +1272,14 @@ static void launch_lds(SL &p, const Grid &g, int NF, int nb, bool res, hipStream
 #undef CASE
       default: throw Error(1, "error in kslaplacian_r! This subroutine is for nf in 1-8.");
     }
+  } else if (!p.out) {  // partials of <in|out> only
+    if (!p.dotp || p.cmax || p.omax || p.accumulate) throw Error(1, "stencil: nothing to compute");
+    switch (NF) {
+#define CASE(N) case N: launch_lds_nf<N, 7>(p, L, nb, s); break;
+      CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+#undef CASE
+      default: throw Error(1, "error in kslaplacian_r! This subroutine is for nf in 1-8.");
+    }
   } else if (p.cmax) {  // plain with column maxima
     if (p.dotp) throw Error(1, "stencil: maxima and partials in one launch");
     switch (NF) {
@@ -1245,7 +1359,7 @@ void launch_stencil(const StencilCall &c, hipStream_t s) {
       q.in2 = c.in2; q.ca = c.ca; q.cb = c.cb; q.dotp2 = c.dot_partial2; q.hin = c.hin;
     }
     if (c.tag) {  // band arrays read and written: in (+ in2 + H in2) and out
-      const double arrays = c.ca ? (c.in2 ? 4.0 : 3.0) : 2.0;
+      const double arrays = c.ca ? (c.in2 ? 4.0 : 3.0) : c.out ? 2.0 : 1.0;
       Timed t(c.tag, 8.0 * ((double)c.nb * arrays * g.n() + (c.veff ? g.n() : 0)));
       launch_lds(q, g, nf, c.nb, false, s);
     } else {
@@ -1269,7 +1383,7 @@ void launch_stencil(const StencilCall &c, hipStream_t s) {
     }
     return;
   }
-  if (c.ca) throw Error(1, "stencil: the combination form runs on the tiled path only");
+  if (c.ca || !c.out) throw Error(1, "stencil: this form runs on the tiled path only");
   if (c.in_max || c.out_max || c.expand_max || c.norm_partial)
     throw Error(1, "stencil: norm and max outputs run on the tiled path only");
   p.zc = 8;
@@ -1480,9 +1594,37 @@ void launch_precond_resid(const Grid &g, const double *h, const double *sp, long
   HIPCK(hipGetLastError());
 }
 
+// The matrix-core gather where it is the faster one: at least 8 bands to fill its 16 columns; one
+// table of up to 9 projectors only for up to 8 GB of bands (64x60x66 x 100: 58 -> 46 us per
+// pass, 96^3 x 512: 0.70 -> 0.59 ms, but 128^3 x 1024: 2.6 -> 2.9 ms, where 16 bands per
+// work-group are spread over too many pages).  Four tables in one pass: 96^3 x 256 x 32 atoms
+// 0.82 -> 0.25 ms.
+static bool gather_mfma(const NonlocalPlan &pl, GatherArgs g, const double *psi, long ld, int nb, long ld_out,
+                        bool accumulate, hipStream_t s) {
+  const int rt = (g.ntab * pl.max_iprj + 15) / 16;
+  if (param("gather_mfma", 1.0) < 1.0 || nb < 8 || pl.nact > 65535 || pl.max_iprj > 32 || rt > 8) return false;
+  if (g.ntab == 1 && pl.max_iprj <= 9 && ld * nb > (1L << 30)) return false;
+  Timed t("nl_gather", 8.0 * ((double)nb * pl.nent + (double)g.ntab * pl.nprjmx * pl.nent));
+  g.act = pl.act; g.lst = pl.lst; g.num_list = pl.num_list; g.nprjmx = pl.nprjmx; g.nb = nb;
+  g.psi = psi; g.ld = ld; g.ld_out = ld_out; g.accumulate = accumulate ? 1 : 0;
+  const dim3 grid(nblk(nb, 16), pl.nact);
+  switch (rt) {
+#define CASE(N) case N: hipLaunchKernelGGL(k_gather_mfma<N>, grid, dim3(256), 0, s, g); break;
+    CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
+#undef CASE
+  }
+  HIPCK(hipGetLastError());
+  return true;
+}
+
 void launch_gather(const NonlocalPlan &pl, const double *psi, long ld, int nb, double *rp,
                    long ld_rp, bool accumulate, hipStream_t s) {
   if (pl.nact == 0 || nb == 0) return;
+  GatherArgs g{};
+  g.ntab = 1;
+  g.tab[0] = pl.vnl;
+  g.out[0] = rp;
+  if (gather_mfma(pl, g, psi, ld, nb, ld_rp, accumulate, s)) return;
   Timed t("nl_gather", 8.0 * ((double)nb * pl.nent + (double)pl.nprjmx * pl.nent));
   const bool bm = param("nl_gather_band_major", 1.0) >= 1.0 && pl.nact <= 65535;
   auto grid = [&](unsigned groups) { return bm ? dim3(groups, pl.nact) : dim3(pl.nact, groups); };
@@ -1498,6 +1640,26 @@ void launch_gather(const NonlocalPlan &pl, const double *psi, long ld, int nb, d
     throw Error(1, "nonlocal projectors: more than 32 per atom are not supported");
   }
   HIPCK(hipGetLastError());
+}
+
+void launch_gather4(const NonlocalPlan &pl, const double *dvnl, const double *psi, long ld, int nb, double *rp,
+                    double *drp, long n1, hipStream_t s) {
+  if (pl.nact == 0 || nb == 0) return;
+  const long tab = (long)pl.num_list * pl.nprjmx * pl.num_ppcell;
+  GatherArgs g{};
+  g.ntab = 4;
+  g.tab[0] = pl.vnl;
+  g.out[0] = rp;
+  for (int d = 0; d < 3; d++) {
+    g.tab[1 + d] = dvnl + d * tab;
+    g.out[1 + d] = drp + (long)d * n1 * nb;
+  }
+  if (gather_mfma(pl, g, psi, ld, nb, n1, false, s)) return;
+  for (int d = 0; d < 4; d++) {  // a pass over psi per table
+    NonlocalPlan pd = pl;
+    pd.vnl = g.tab[d];
+    launch_gather(pd, psi, ld, nb, g.out[d], n1, false, s);
+  }
 }
 
 void launch_coef(const NonlocalPlan &pl, const double *rp, long ld_rp, int nb, const double *X,

@@ -240,6 +240,10 @@ void launch_precond_resid(const Grid &g, const double *h, const double *sp, long
 // <p|psi>: rp(i, slot, b) (=|+=) sum_k vnl(k,i,slot) psi_b(lst(k,slot)-1)
 void launch_gather(const NonlocalPlan &pl, const double *psi, long ld, int nb, double *rp,
                    long ld_rp, bool accumulate, hipStream_t s);
+// <p|psi> and <d p/d R_x,y,z|psi> in one pass: rp from pl's table, drp (3 arrays of n1 x nb, n1 =
+// nprjmx num_ppcell) from the three tables dvnl of the same shape and lists
+void launch_gather4(const NonlocalPlan &pl, const double *dvnl, const double *psi, long ld, int nb, double *rp,
+                    double *drp, long n1, hipStream_t s);
 // coef(j, slot, b) = sum_i rp(i, slot, b) X(i, j; atom) / dV, X = dij(:,:,ns,na) or sss(:,:,1,ispe)
 void launch_coef(const NonlocalPlan &pl, const double *rp, long ld_rp, int nb, const double *X,
                  bool use_sss, int ns, double dvinv, double *coef, long ld_coef, hipStream_t s,

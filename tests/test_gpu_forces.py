@@ -37,3 +37,45 @@ def test_force_eig_edges(kk, orc, nprj, nf, nperi, bands, atoms):
         call("force_eig_r", **kw, **arr, fatx=f[0], faty=f[1], fatz=f[2])
         out.append(np.stack(f))
     np.testing.assert_allclose(out[0], out[1], rtol=0, atol=1e-11 * np.abs(out[1]).max())
+
+
+@pytest.mark.parametrize("nprj", [1, 9, 16, 18, 32])
+@pytest.mark.parametrize("bands,n", [(7, 12), (8, 12), (17, 11), (40, 14)])
+def test_gather_edges(kk, nprj, bands, n):
+    """<p|psi> of a band block (orthogonalization_r's rspsep at nflag = 1, one pass over all
+    bands) and the adjoint's four-table pass against numpy: fewer bands than the matrix-core
+    kernel takes, ragged band and projector counts, lists that end inside a 16-point step.  Each
+    value is a sum of natinf products: off by at most natinf 2^-53 times their absolute sum."""
+    s = synth.make_system(n, 0.4, 3, bands, seed=nprj + bands)
+    rng = np.random.default_rng(nprj)
+    tabs = [np.asfortranarray(rng.standard_normal((s.num_list, nprj, s.natom))) for _ in range(4)]
+    dij = rng.standard_normal((nprj, nprj, 1, s.natom))
+    dij = np.asfortranarray(dij + dij.transpose(1, 0, 2, 3))
+    f = rng.random(bands)
+    kw = synth.abi_args(s, nprjmx=nprj, nprj=np.array([nprj], dtype=np.int32), vnlocp=tabs[0], dij=dij)
+    psi = synth.random_bands(s)
+    dedv, dedr = np.zeros(s.npts), np.zeros((s.natom, 3), order="F")
+    kk.call("energy_adjoint_r", **kw, dvnlocp=np.asfortranarray(np.stack(tabs[1:], axis=-1)), svecre=psi, fnele=f,
+            dedv=dedv, dedr=dedr)
+    want, bound = np.zeros((s.natom, 3)), np.zeros((s.natom, 3))
+    for a in range(s.natom):
+        m = s.natinf[a]
+        w = psi[s.lstvec2[:m, a] - 1]
+        r = [t[:m, :, a].T @ w for t in tabs]
+        ra = [np.abs(t[:m, :, a]).T @ np.abs(w) for t in tabs]
+        for d in range(3):
+            want[a, d] = 2 * np.einsum("l,il,ij,jl->", f, r[1 + d], dij[:, :, 0, a], r[0], optimize=True)
+            bound[a, d] = 2 * np.einsum("l,il,ij,jl->", f, ra[1 + d], np.abs(dij[:, :, 0, a]), ra[0], optimize=True)
+    eps = (2 * s.num_list + nprj * nprj + bands) * 2.0 ** -53
+    assert np.all(np.abs(dedr - want) <= eps * bound)
+    np.testing.assert_allclose(dedv, s.dv * (f * psi * psi).sum(axis=1), rtol=bands * 2.0 ** -52)
+    # the one-table pass: <p|psi> of the orthonormal bands it returns
+    rp = np.zeros((nprj, s.natom, bands), order="F")
+    kk.call("orthogonalization_r", **dict(kw, sss=np.zeros((nprj, nprj, 1), order="F")), nflag=1, svecre=psi,
+            ssvre=psi, rspsep=rp)
+    kappa = 50.0  # of the triangular factor applied to psi and to <p|psi> alike
+    for a in range(s.natom):
+        m = s.natinf[a]
+        w = psi[s.lstvec2[:m, a] - 1]
+        err = np.abs(rp[:, a] - tabs[0][:m, :, a].T @ w)
+        assert np.all(err <= kappa * (s.num_list + s.npts) * 2.0 ** -53 * (np.abs(tabs[0][:m, :, a]).T @ np.abs(w)))
