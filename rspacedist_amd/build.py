@@ -13,7 +13,7 @@ LIB = os.path.join(HERE, "libkukan_hip.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 HIPCC = os.path.join(ROCM, "bin", "hipcc")
 ARCH = "gfx950"
-SOURCES = ["common.hip", "kernels.hip", "gemm_mixed.hip", "gemm_f64.hip", "hartree_cg.hip", "solvers.hip", "batch.hip", "abi.hip",
+SOURCES = ["common.hip", "kernels.hip", "gemm_mixed.hip", "gemm_f64.hip", "hartree_cg.hip", "seqcg.hip", "solvers.hip", "batch.hip", "abi.hip",
            "noalloc.hip", "bloch.hip", "abi_bloch.hip", "transfer.hip", "abi_trans.hip", "checkpoint.hip", "projector.hip",
            "force.hip"]
 CFLAGS = ["-O3", "-fPIC", "-std=c++17", f"--offload-arch={ARCH}", "-Wall", "-Wno-unused-result",

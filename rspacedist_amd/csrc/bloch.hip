@@ -12,10 +12,9 @@
 // table per call, the gather <p|u> = sum vnlocp e^{i k.x} u and the owner-computes expansion
 // sum e^{-i k.x} vnlocp c over the same CSR plan as the real path.
 //
-// Solvers: kscg_c band by band as kscg8f.F90:492-1032 (device kernels, per-band scalars on
-// the host), orthogonalization_c as Cholesky-QR (rocBLAS zgemm, rocSOLVER zpotrf, ztrsm: the
-// Gram-Schmidt Q), single-band Gram-Schmidt with zgemv, rayleighritz_c with zgemm and
-// rocSOLVER zheevd.
+// Solvers: kscg_c band by band as kscg8f.F90:492-1032 (seqcg.hip), orthogonalization_c as
+// Cholesky-QR (rocBLAS zgemm, rocSOLVER zpotrf, ztrsm: the Gram-Schmidt Q), single-band
+// Gram-Schmidt with zgemv, rayleighritz_c with zgemm and rocSOLVER zheevd.
 #include <rocblas/rocblas.h>
 #include <rocsolver/rocsolver.h>
 
@@ -28,6 +27,7 @@
 #include "kukan_internal.hpp"
 #include "solvers.hpp"
 #include "bloch.hpp"
+#include "seqcg.hpp"
 
 namespace kukan {
 namespace {
@@ -245,14 +245,6 @@ __global__ void k_zdot_red(const zt *part, int np, double scale, zt *res) {
   res[b] = zsc(scale, s);
 }
 
-// out = a x + c y (complex scalars; y may be null)
-__global__ void k_zaxpby(long n, zt a, const zt *x, zt c, const zt *y, zt *out) {
-  const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  zt v = zmul(a, x[i]);
-  if (y) v = zadd(v, zmul(c, y[i]));
-  out[i] = v;
-}
 // per-band real scale
 __global__ void k_zscale(long n, double s, zt *x) {
   const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
@@ -487,12 +479,6 @@ zc ZCtx::dot1(const zt *x, const zt *y, double scale) {
   return zc(h.x, h.y);
 }
 
-void ZCtx::axpby(long len, zc a, const zt *x, zc b, const zt *y, zt *out) {
-  hipLaunchKernelGGL(k_zaxpby, dim3(nb_(len, 256)), dim3(256), 0, c.s, len, zmk(a.real(), a.imag()), x,
-                     zmk(b.real(), b.imag()), y, out);
-  HIPCK(hipGetLastError());
-}
-
 void ZCtx::scale(long len, double s, zt *x) {
   hipLaunchKernelGGL(k_zscale, dim3(nb_(len, 256)), dim3(256), 0, c.s, len, s, x);
   HIPCK(hipGetLastError());
@@ -629,127 +615,14 @@ void zrayleigh_ritz(ZCtx &z, int M, const double *veff, bool l_rrb, zt *psi, zt 
   }
 }
 
-// kscg_c band by band (kscg8f.F90:492-1032; per-band scalars on the host)
+// kscg_c band by band (kscg8f.F90:492-1032)
 void zkscg_c(ZCtx &z, int M, int northo, int nkscg, int nsdmax, int nprecon_cg, int key_cmpt,
              int key_nocmpt, double epssd, const double *veff, zt *Psi, zt *SPsi, zt *Cps, zt *H,
              double *sval, double *resid, int *ksconv, int *ksitmax) {
-  Ctx &c = z.c;
-  const long n = z.n(), n1 = z.n1();
-  const double dv = c.g.dv();
-  rocblas_handle h = lib().blas;
-  zt *rvec = z.zbuf("zcg.rvec", n), *pvec = z.zbuf("zcg.pvec", n), *pv = z.zbuf("zcg.pv", n);
-  zt *rv = z.zbuf("zcg.rv", n), *spv = z.zbuf("zcg.spv", n), *av = z.zbuf("zcg.av", n);
-  zt *asv = z.zbuf("zcg.asv", n), *avc = z.zbuf("zcg.avc", M);
-  zt *crp = z.zbuf("zcg.crp", n1), *cpp = z.zbuf("zcg.cpp", n1), *cp = z.zbuf("zcg.cp", n1);
-  const bool same_s = c.q_zero && SPsi == Psi;
   const int key = northo == 2 ? key_cmpt : key_nocmpt;
-  const rocblas_double_complex rdv(dv, 0.0), zero(0.0, 0.0), one(1.0, 0.0), mone(-1.0, 0.0);
-  // eigenvalue and residual estimates are host scalars here: collected on the host, stored once
-  std::vector<double> hsv(M), hres(M);
-  HIPCK(hipMemcpyAsync(hsv.data(), sval, sizeof(double) * M, hipMemcpyDeviceToHost, c.s));
-  HIPCK(hipMemcpyAsync(hres.data(), resid, sizeof(double) * M, hipMemcpyDeviceToHost, c.s));
-  sync();
-  auto zero_n = [&](zt *x, long len) { HIPCK(hipMemsetAsync(x, 0, sizeof(zt) * std::max<long>(1, len), c.s)); };
-  auto copy = [&](zt *dst, const zt *src, long len) {
-    if (len > 0) HIPCK(hipMemcpyAsync(dst, src, sizeof(zt) * len, hipMemcpyDeviceToDevice, c.s));
-  };
-  // x -= Psi(:, 0..l) dV <S psi_j|x> (kscg8f.F90:751-778)
-  auto project = [&](int l, zt *x, zt *sx, zt *cx) {
-    BLASCK(rocblas_zgemv(h, rocblas_operation_conjugate_transpose, (int)n, l + 1, &rdv,
-                         (const rocblas_double_complex *)SPsi, (int)n, (const rocblas_double_complex *)x, 1,
-                         &zero, (rocblas_double_complex *)avc, 1));
-    BLASCK(rocblas_zgemv(h, rocblas_operation_none, (int)n, l + 1, &mone, (const rocblas_double_complex *)Psi,
-                         (int)n, (const rocblas_double_complex *)avc, 1, &one, (rocblas_double_complex *)x, 1));
-    if (sx)
-      BLASCK(rocblas_zgemv(h, rocblas_operation_none, (int)n, l + 1, &mone,
-                           (const rocblas_double_complex *)SPsi, (int)n, (const rocblas_double_complex *)avc,
-                           1, &one, (rocblas_double_complex *)sx, 1));
-    if (cx && n1 > 0)
-      BLASCK(rocblas_zgemv(h, rocblas_operation_none, (int)n1, l + 1, &mone,
-                           (const rocblas_double_complex *)Cps, (int)n1, (const rocblas_double_complex *)avc,
-                           1, &one, (rocblas_double_complex *)cx, 1));
-  };
-  for (int l = 0; l < M; l++) {
-    zt *psi = Psi + n * l, *spsi = SPsi + n * l, *hp = H + n * l, *cps = Cps + n1 * l;
-    for (int loop = 0; loop < northo; loop++) zortho_c_01(z, M, l + 1, key, key_cmpt, Psi, SPsi, Cps);
-    copy(cp, cps, n1);
-    z.hpsi(veff, psi, n, 1, cp, n1, hp, n);
-    int iiter = 0;
-    bool conv = false;
-    zc r1r, r2r(0.0, 0.0);
-    while (iiter < nsdmax && !conv) {
-      iiter++;
-      bool doreset = (iiter == 1) || (iiter == 10) || ((iiter - 1) % 200 == 0);
-      if (doreset) {
-        r2r = zc(1.0, 0.0);
-        zero_n(pvec, n); zero_n(rvec, n); zero_n(pv, n); zero_n(spv, n);
-        if (n1 > 0) zero_n(cpp, n1);
-      }
-      r1r = r2r;
-      const double valre = z.dot1(psi, hp, dv).real();
-      hsv[l] = valre;
-      z.axpby(n, zc(-1.0, 0.0), hp, zc(valre, 0.0), spsi, rvec);  // r = -(H psi - eps S psi)
-      if (nprecon_cg == 1) z.precond(rvec, rv);
-      else copy(rv, rvec, n);
-      for (int loop = 0; loop < northo; loop++) project(l, rv, nullptr, nullptr);
-      z.proj(rv, n, 1, cp, n1);
-      copy(crp, cp, n1);
-      if (same_s) copy(asv, rv, n);
-      else z.spsi(rv, n, 1, crp, n1, asv, n);
-      r2r = z.dot1(rv, rvec, dv);  // sum conj(K r) r (orthogonalization_c_04(v1 = r, v2 = K r))
-      const double res = std::abs(r2r);
-      hres[l] = res;
-      if (nkscg == 1) {
-        const double a2 = std::abs(r1r);
-        const zc t = std::conj(r1r) * r2r / (a2 * a2);  // kscg_c_03
-        z.axpby(n, zc(1.0, 0.0), rv, t, pv, pv);
-        copy(pvec, pv, n);
-        z.axpby(n, zc(1.0, 0.0), asv, t, spv, spv);
-        if (n1 > 0) z.axpby(n1, zc(1.0, 0.0), crp, r2r / r1r, cpp, cpp);
-      } else {
-        copy(pvec, rv, n);
-        copy(spv, asv, n);
-        copy(cpp, crp, n1);
-      }
-      copy(cp, cpp, n1);
-      copy(asv, spv, n);
-      for (int loop = 0; loop < northo; loop++) project(l, pvec, asv, cp);
-      const double vecnor = z.dot1(pvec, asv, dv).real();
-      if (vecnor <= 0.0) throw Error(2, "kscg_c: pvec has negative norm");
-      const double tn = 1.0 / std::sqrt(vecnor);
-      z.scale(n, tn, pvec);
-      z.scale(n, tn, asv);
-      if (n1 > 0) z.scale(n1, tn, cp);
-      z.hpsi(veff, pvec, n, 1, cp, n1, av, n);
-      const double pap = z.dot1(pvec, av, dv).real();
-      const zc sap = z.dot1(psi, av, dv);
-      // kscg_c_05 (kscg8f.F90:1233-1274)
-      const double eps = 1.0e-14, s2 = std::norm(sap);
-      const double gamma = (valre + pap) * 0.5 - std::sqrt((valre - pap) * (valre - pap) * 0.25 + s2);
-      double alph;
-      zc cbeta;
-      if (std::fabs((valre - gamma) / gamma) > eps) {
-        const double d = std::sqrt(s2 + (valre - gamma) * (valre - gamma));
-        const zc calph = sap / d;
-        cbeta = zc(-(valre - gamma) / d, 0.0);
-        alph = std::abs(calph);
-        if (alph > eps) cbeta = cbeta * alph / calph;
-      } else {
-        alph = 1.0;
-        cbeta = zc(0.0, 0.0);
-      }
-      z.axpby(n, zc(alph, 0.0), psi, cbeta, pvec, psi);
-      z.axpby(n, zc(alph, 0.0), hp, cbeta, av, hp);
-      if (!same_s) z.axpby(n, zc(alph, 0.0), spsi, cbeta, asv, spsi);
-      if (n1 > 0) z.axpby(n1, zc(alph, 0.0), cps, cbeta, cp, cps);
-      conv = std::sqrt(res) < epssd;
-      *ksconv = *ksconv && (conv || iiter < nsdmax);
-    }
-    *ksitmax = std::max(*ksitmax, iiter);
-  }
-  HIPCK(hipMemcpyAsync(sval, hsv.data(), sizeof(double) * M, hipMemcpyHostToDevice, c.s));
-  HIPCK(hipMemcpyAsync(resid, hres.data(), sizeof(double) * M, hipMemcpyHostToDevice, c.s));
-  sync();
+  SeqCgArgs<zt> q{M, northo, nkscg, nsdmax, nprecon_cg, z.ns_h, key == key_cmpt, epssd,
+                  veff, Psi, SPsi, H, Cps, sval, resid, ksconv, ksitmax};
+  seq_cg(z, q);
 }
 
 namespace {

@@ -41,8 +41,6 @@ struct ZCtx {
   void dots(const double2 *x, long ldx, const double2 *y, long ldy, int nb, double2 *res,
             double scale);
   std::complex<double> dot1(const double2 *x, const double2 *y, double scale);
-  void axpby(long len, std::complex<double> a, const double2 *x, std::complex<double> b,
-             const double2 *y, double2 *out);
   void scale(long len, double s, double2 *x);
 };
 

@@ -15,6 +15,7 @@
 #include "hartree_cg.hpp"
 #include "kukan_internal.hpp"
 #include "solvers.hpp"
+#include "seqcg.hpp"
 
 namespace kukan {
 namespace {
@@ -1326,102 +1327,10 @@ void rayleigh_ritz(Ctx &c, int M, int ns, const double *veffs, bool l_rrb, doubl
 // ============================================================================= kscg_r
 // Band-sequential preconditioned CG exactly as kscg8f.F90:98-472.
 void kscg_sequential(Ctx &c, const KscgArgs &a) {
-  const long n = c.g.n(), n1 = (long)c.pl.nprjmx * c.pl.num_ppcell;
-  const int M = a.neigmx;
-  rocblas_handle h = lib().blas;
-  double *rvecre = c.buf("cg.rvecre", n), *pvecre = c.buf("cg.pvecre", n), *pvre = c.buf("cg.pvre", n);
-  double *rvre = c.buf("cg.rvre", n), *spvre = c.buf("cg.spvre", n), *avre = c.buf("cg.avre", n);
-  double *asvre = c.buf("cg.asvre", n);
-  double *rrpsep = c.buf("cg.rrpsep", std::max<long>(1, n1)), *rppsep = c.buf("cg.rppsep", std::max<long>(1, n1));
-  double *rpsep = c.buf("cg.rpsep", std::max<long>(1, n1));
-  double *avreal = c.buf("cg.avreal", M);
-  // device scalars: 0 r1rr, 1 r2rr, 2 pap, 3 sapre, 4 vecnor, 5 tmp, 6 alph, 7 beta, 8 t, 9 eps
-  double *sc = c.buf("cg.sc", 16);
-  const double dv = c.g.dv(), zero = 0.0, one = 1.0, mone = -1.0;
   const int key = a.northo == 2 ? a.key_cmpt : a.key_nocmpt;
-  std::vector<double> res_h(1);
-  c.clear_flag(1);
-  for (int l = 0; l < M; l++) {
-    double *psi = a.psi + n * l, *spsi = a.spsi + n * l, *hp = a.hpsi + n * l, *rps = a.rsp + n1 * l;
-    for (int loop = 0; loop < a.northo; loop++) ortho_r_01(c, M, l + 1, key, a.key_cmpt, a.psi, a.spsi, a.rsp);
-    if (n1 > 0) HIPCK(hipMemcpyAsync(rpsep, rps, sizeof(double) * n1, hipMemcpyDeviceToDevice, c.s));
-    c.hpsi(a.ns, a.veffs, psi, n, 1, rpsep, n1, hp, n, false, nullptr);
-    int iiter = 0;
-    bool conv = false;
-    while (iiter < a.nsdmax && !conv) {
-      iiter++;
-      bool doreset = (iiter == 1) || (iiter == 10) || ((iiter - 1) % 200 == 0);
-      if (doreset) {
-        launch_fill(1, 1.0, sc + 1, c.s);
-        launch_fill(n, 0.0, pvecre, c.s);
-        launch_fill(n, 0.0, rvecre, c.s);
-        launch_fill(n, 0.0, pvre, c.s);
-        launch_fill(n, 0.0, spvre, c.s);
-        if (n1 > 0) launch_fill(n1, 0.0, rppsep, c.s);
-      }
-      HIPCK(hipMemcpyAsync(sc + 0, sc + 1, sizeof(double), hipMemcpyDeviceToDevice, c.s));
-      double *ev = a.sval + l;
-      c.dots(psi, n, hp, n, 1, ev);
-      // r = -(h - eps s)
-      launch_axpby(n, 1, nullptr, -1.0, hp, n, ev, 1.0, spsi, n, rvecre, n, c.s);
-      if (a.nprecon_cg == 1) launch_precond(c.g, rvecre, n, false, 1, rvre, n, 1, c.s);
-      else HIPCK(hipMemcpyAsync(rvre, rvecre, sizeof(double) * n, hipMemcpyDeviceToDevice, c.s));
-      for (int loop = 0; loop < a.northo; loop++) {
-        BLASCK(rocblas_dgemv(h, rocblas_operation_transpose, (int)n, l + 1, &dv, a.spsi, (int)n, rvre,
-                             1, &zero, avreal, 1));
-        BLASCK(rocblas_dgemv(h, rocblas_operation_none, (int)n, l + 1, &mone, a.psi, (int)n, avreal, 1,
-                             &one, rvre, 1));
-      }
-      c.proj(rvre, n, 1, rpsep, n1);
-      if (n1 > 0) HIPCK(hipMemcpyAsync(rrpsep, rpsep, sizeof(double) * n1, hipMemcpyDeviceToDevice, c.s));
-      c.spsi(rvre, n, 1, rrpsep, n1, asvre, n);
-      c.dots(rvecre, n, rvre, n, 1, sc + 1);
-      HIPCK(hipMemcpyAsync(a.resid + l, sc + 1, sizeof(double), hipMemcpyDeviceToDevice, c.s));
-      if (a.nkscg == 1) {
-        hipLaunchKernelGGL(k_ratio, dim3(1), dim3(64), 0, c.s, 1, sc + 1, sc + 0, 0, sc + 8);
-        launch_axpby(n, 1, nullptr, 1.0, rvre, n, sc + 8, 1.0, pvre, n, pvre, n, c.s);
-        HIPCK(hipMemcpyAsync(pvecre, pvre, sizeof(double) * n, hipMemcpyDeviceToDevice, c.s));
-        launch_axpby(n, 1, nullptr, 1.0, asvre, n, sc + 8, 1.0, spvre, n, spvre, n, c.s);
-        if (n1 > 0) launch_axpby(n1, 1, nullptr, 1.0, rrpsep, n1, sc + 8, 1.0, rppsep, n1, rppsep, n1, c.s);
-      } else {
-        HIPCK(hipMemcpyAsync(pvecre, rvre, sizeof(double) * n, hipMemcpyDeviceToDevice, c.s));
-        HIPCK(hipMemcpyAsync(spvre, asvre, sizeof(double) * n, hipMemcpyDeviceToDevice, c.s));
-        if (n1 > 0) HIPCK(hipMemcpyAsync(rppsep, rrpsep, sizeof(double) * n1, hipMemcpyDeviceToDevice, c.s));
-      }
-      if (n1 > 0) HIPCK(hipMemcpyAsync(rpsep, rppsep, sizeof(double) * n1, hipMemcpyDeviceToDevice, c.s));
-      HIPCK(hipMemcpyAsync(asvre, spvre, sizeof(double) * n, hipMemcpyDeviceToDevice, c.s));
-      for (int loop = 0; loop < a.northo; loop++) {
-        BLASCK(rocblas_dgemv(h, rocblas_operation_transpose, (int)n, l + 1, &dv, a.spsi, (int)n,
-                             pvecre, 1, &zero, avreal, 1));
-        BLASCK(rocblas_dgemv(h, rocblas_operation_none, (int)n, l + 1, &mone, a.psi, (int)n, avreal, 1,
-                             &one, pvecre, 1));
-        BLASCK(rocblas_dgemv(h, rocblas_operation_none, (int)n, l + 1, &mone, a.spsi, (int)n, avreal, 1,
-                             &one, asvre, 1));
-        if (n1 > 0)
-          BLASCK(rocblas_dgemv(h, rocblas_operation_none, (int)n1, l + 1, &mone, a.rsp, (int)n1, avreal,
-                               1, &one, rpsep, 1));
-      }
-      c.dots(pvecre, n, asvre, n, 1, sc + 4);
-      hipLaunchKernelGGL(k_rsqrt_norm, dim3(1), dim3(64), 0, c.s, 1, sc + 4, sc + 5, c.flag(1));
-      launch_scale(n, 1, sc + 5, pvecre, n, c.s);
-      launch_scale(n, 1, sc + 5, asvre, n, c.s);
-      if (n1 > 0) launch_scale(n1, 1, sc + 5, rpsep, n1, c.s);
-      c.hpsi(a.ns, a.veffs, pvecre, n, 1, rpsep, n1, avre, n, false, sc + 2);
-      c.dots(psi, n, avre, n, 1, sc + 3);
-      hipLaunchKernelGGL(k_kscg05, dim3(1), dim3(64), 0, c.s, 1, ev, sc + 2, sc + 3, nullptr, sc + 6,
-                         sc + 7);
-      launch_axpby(n, 1, sc + 6, 1.0, psi, n, sc + 7, 1.0, pvecre, n, psi, n, c.s);
-      launch_axpby(n, 1, sc + 6, 1.0, hp, n, sc + 7, 1.0, avre, n, hp, n, c.s);
-      launch_axpby(n, 1, sc + 6, 1.0, spsi, n, sc + 7, 1.0, asvre, n, spsi, n, c.s);
-      if (n1 > 0) launch_axpby(n1, 1, sc + 6, 1.0, rps, n1, sc + 7, 1.0, rpsep, n1, rps, n1, c.s);
-      HIPCK(hipMemcpyAsync(res_h.data(), a.resid + l, sizeof(double), hipMemcpyDeviceToHost, c.s));
-      sync();
-      conv = std::sqrt(res_h[0]) < a.epssd;
-      *a.ksconv = *a.ksconv && (conv || iiter < a.nsdmax);
-    }
-    *a.ksitmax = std::max(*a.ksitmax, iiter);
-  }
-  if (c.read_flag(1)) throw Error(2, "kscg_r: pvec has negative norm");
+  SeqCgArgs<double> q{a.neigmx, a.northo, a.nkscg, a.nsdmax, a.nprecon_cg, a.ns, key == a.key_cmpt, a.epssd,
+                      a.veffs, a.psi, a.spsi, a.hpsi, a.rsp, a.sval, a.resid, a.ksconv, a.ksitmax};
+  seq_cg(c, q);
 }
 
 // Block CG: every band advances at once; the reference's per-band projections against
