@@ -7,8 +7,8 @@
 //
 // Batched mode: every stencil pass of all systems is one persistent launch (the items of all
 // systems in one work list), per-band arithmetic runs as launches over a global band table,
-// the Hartree CG of all systems advances as device-side iteration blocks with per-system stop
-// flags, and the band step and the Hartree block are captured once as HIP graphs and
+// the Hartree CG of all systems advances as device-side iteration blocks of two launches per
+// iteration with per-system stop flags (hartree_cg.hip), and the band step and the Hartree block are captured once as HIP graphs and
 // replayed.  Loop mode runs the same kernels system by system (one launch per system and
 // pass, no graphs): the comparison the batching is measured against.  Both modes compute
 // bit-identical results.  The stencil tile (points per thread) and the persistent grid size
@@ -22,6 +22,7 @@
 #include <string>
 #include <vector>
 
+#include "hartree_cg.hpp"
 #include "kukan_hip.h"
 #include "kukan_internal.hpp"
 #include "solvers.hpp"
@@ -146,13 +147,13 @@ __global__ __launch_bounds__(256) void k_band_update(const BandRef *bands, const
 }
 
 // ------------------------------------------------------------------ batched Hartree CG
-// state[0] = done, state[1] = iterations; sc = {r1r, pap, r2r, mean b}
+// The iteration is that of hartree_cg.hip over all systems (two launches); here are its start and
+// the tables.  state = {done, iteration, iterations taken}, sc = {<r|r> of odd / even iterations,
+// mean b}.
 struct HSys {
-  double *rho, *vh, *b, *r, *p, *ap, *avhs, *sc, *part;
+  double *rho, *vh, *r, *p, *ap, *sc;
   int *state;
   long n;
-  int np;
-  double dvo;
 };
 constexpr int HCH = 64;
 
@@ -165,7 +166,7 @@ __global__ __launch_bounds__(256) void k_hb_sum(const HSys *hs, int which, doubl
   for (long i = i0 + threadIdx.x; i < i1; i += 256) {
     if (which == 0) {
       const double bi = 2.0 * M_PI * H.rho[i];
-      H.b[i] = bi;
+      H.r[i] = bi;
       s += bi;
     } else {
       s += H.r[i] * H.r[i];
@@ -176,96 +177,29 @@ __global__ __launch_bounds__(256) void k_hb_sum(const HSys *hs, int which, doubl
   __syncthreads();
   if (threadIdx.x == 0) part[(long)blockIdx.y * HCH + blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
 }
-__global__ void k_hb_fold(const HSys *hs, int ns, const double *part, int slot, int mean) {
+// mean: sc[2] = mean of the sums; else <r|r> of the start, and the iteration's state
+__global__ void k_hb_fold(const HSys *hs, int ns, const double *part, int mean) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= ns) return;
   double s = 0.0;
   for (int c = 0; c < HCH; c++) s += part[(long)i * HCH + c];
-  hs[i].sc[slot] = mean ? s / (double)hs[i].n : s;
-  if (slot == 0) {
+  hs[i].sc[mean ? 2 : 1] = mean ? s / (double)hs[i].n : s;
+  if (!mean) {
     hs[i].state[0] = 0;
-    hs[i].state[1] = 0;
+    hs[i].state[1] = 1;
+    hs[i].state[2] = 0;
   }
 }
-// b -= mean ; avhs = A v (in ap) ; r = b - avhs ; p = r
+// r = b - mean - A v (A v in ap, b in r); p = r
 __global__ __launch_bounds__(256) void k_hb_init(const HSys *hs) {
   const HSys H = hs[blockIdx.y];
-  const double m = H.sc[3];
+  const double m = H.sc[2];
   const long stride = (long)gridDim.x * 256;
   for (long i = blockIdx.x * 256L + threadIdx.x; i < H.n; i += stride) {
-    const double bi = H.b[i] - m;
-    H.b[i] = bi;
-    H.avhs[i] = H.ap[i];
-    const double ri = bi - H.ap[i];
+    const double ri = H.r[i] - m - H.ap[i];
     H.r[i] = ri;
     H.p[i] = ri;
   }
-}
-__global__ void k_hb_begin(const HSys *hs, int ns, int *alldone) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) *alldone = 1;
-  if (i >= ns) return;
-  const HSys H = hs[i];
-  if (H.state[0]) return;
-  H.state[1] += 1;
-  if (H.state[1] > 1) H.sc[0] = H.sc[2];
-}
-__global__ void k_hb_pap(const HSys *hs, int ns) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ns) return;
-  const HSys H = hs[i];
-  if (H.state[0]) return;
-  double s = 0.0;
-  for (int c = 0; c < H.np; c++) s += H.part[c];
-  H.sc[1] = s;
-}
-__global__ __launch_bounds__(256) void k_hb_update(const HSys *hs, double *part) {
-  __shared__ double red[4];
-  const HSys H = hs[blockIdx.y];
-  if (H.state[0]) return;
-  const double alph = H.sc[0] / H.sc[1];
-  const long chunk = (H.n + HCH - 1) / HCH;
-  const long i0 = blockIdx.x * chunk, i1 = min(H.n, i0 + chunk);
-  double s = 0.0;
-  for (long i = i0 + threadIdx.x; i < i1; i += 256) {
-    H.vh[i] = H.vh[i] + alph * H.p[i];
-    H.avhs[i] = H.avhs[i] + alph * H.ap[i];
-    const double ri = H.b[i] - H.avhs[i];
-    H.r[i] = ri;
-    s += ri * ri;
-  }
-  for (int off = 32; off > 0; off >>= 1) s += __shfl_down(s, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-  __syncthreads();
-  if (threadIdx.x == 0) part[(long)blockIdx.y * HCH + blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
-}
-__global__ void k_hb_r2r(const HSys *hs, int ns, const double *part) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ns) return;
-  const HSys H = hs[i];
-  if (H.state[0]) return;
-  double s = 0.0;
-  for (int c = 0; c < HCH; c++) s += part[(long)i * HCH + c];
-  H.sc[2] = s;
-}
-__global__ __launch_bounds__(256) void k_hb_dir(const HSys *hs, int ncgres) {
-  const HSys H = hs[blockIdx.y];
-  if (H.state[0]) return;
-  const double beta = (H.state[1] % ncgres == 0) ? 0.0 : H.sc[2] / H.sc[0];
-  const long stride = (long)gridDim.x * 256;
-  for (long i = blockIdx.x * 256L + threadIdx.x; i < H.n; i += stride) H.p[i] = H.r[i] + beta * H.p[i];
-}
-__global__ void k_hb_check(const HSys *hs, int ns, double eps, int ncgmin, int ncgmax,
-                           int *alldone) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ns) return;
-  const HSys H = hs[i];
-  if (!H.state[0]) {
-    const int loop = H.state[1];
-    const double dp = sqrt(H.sc[2] * H.dvo);
-    if (loop >= ncgmin && (loop >= ncgmax || dp <= eps)) H.state[0] = 1;
-  }
-  if (!H.state[0]) atomicAnd(alldone, 0);
 }
 
 inline unsigned nb_(long n, int t) { return (unsigned)((n + t - 1) / t); }
@@ -409,10 +343,8 @@ struct BatchSystem {
          *p = nullptr, *hp = nullptr, *rp = nullptr, *coef = nullptr, *part = nullptr,
          *ones = nullptr;
   int *lst = nullptr;
-  double *rho = nullptr, *vh = nullptr, *hb = nullptr, *hr = nullptr, *hpv = nullptr,
-         *hap = nullptr, *havhs = nullptr, *hsc = nullptr, *hpart = nullptr;
-  int *hstate = nullptr;
-  long nparts = 0, sparts = 0, hparts = 0;
+  double *rho = nullptr, *vh = nullptr, *hr = nullptr, *hpv = nullptr, *hpw = nullptr, *hap = nullptr;
+  long nparts = 0, sparts = 0;
   std::vector<void *> owned;
   template <class T>
   T *alloc(size_t count) {
@@ -433,12 +365,17 @@ struct Batch {
   double *bpart = nullptr, *eps = nullptr, *d = nullptr, *pp = nullptr, *sap = nullptr,
          *pap = nullptr, *ab = nullptr, *sval = nullptr, *hpart = nullptr;
   HSys *hs = nullptr;
-  int *alldone = nullptr;
+  double *hsc = nullptr;     // 3 per system
+  int *hstate = nullptr;     // 3 per system
+  std::vector<HcgArgs> hcg;  // the Hartree iteration's arguments, their device copy and units
+  HcgArgs *hcg_dev = nullptr;
+  int2 *hdir = nullptr, *hupd = nullptr;
+  std::vector<int> hd0, hu0;  // each system's first unit (ns + 1)
   std::vector<void *> owned;
   bool ready = false;
   int P = 2, grid = 1024;
-  // plans over all systems [0] and per system [1 + i]; kinds: H psi, H p, precond, Hartree
-  std::vector<StencilBatchPlan> plan[5];
+  // plans over all systems [0] and per system [1 + i]; kinds: H psi, H p, precond, A v
+  std::vector<StencilBatchPlan> plan[4];
   hipGraphExec_t g_band = nullptr, g_hart = nullptr;
   int hart_blk = 16;
   // orthonormalisation: per-system descriptors and unit tables (system-major) with each
@@ -488,9 +425,6 @@ StencilCall call_for(BatchSystem &S, int kind, const double *eps_band) {
     c.dot_ld = S.nparts;
   } else if (kind == 2) {  // K r with r = -(H psi - eps psi)
     c.in = S.hpsi; c.in2 = S.psi; c.eps = eps_band; c.sign = -1.0; c.out = S.p;
-  } else if (kind == 3) {  // Hartree: A p with <p|A p> partials, skipped once converged
-    c.in = S.hpv; c.out = S.hap; c.nb = 1; c.nfh_coeffs = 4; c.dot_partial = S.hpart;
-    c.dot_ld = S.hparts; c.skip = S.hstate;
   } else {  // Hartree start: A v
     c.in = S.vh; c.out = S.hap; c.nb = 1; c.nfh_coeffs = 4;
   }
@@ -499,7 +433,7 @@ StencilCall call_for(BatchSystem &S, int kind, const double *eps_band) {
 
 void build_plans(Batch &B) {
   const int ns = (int)B.sys.size();
-  for (int kind = 0; kind < 5; kind++) {
+  for (int kind = 0; kind < 4; kind++) {
     B.plan[kind].clear();
     std::vector<StencilCall> all;
     for (int i = 0; i < ns; i++) all.push_back(call_for(*B.sys[i], kind, B.eps + B.sys[i]->band0));
@@ -585,58 +519,50 @@ void hartree_start(Batch &B, int s0, int s1, bool batched, hipStream_t s) {
   HSys *hs = B.hs + s0;
   double *part = B.hpart + (long)s0 * HCH;
   hipLaunchKernelGGL(k_hb_sum, dim3(HCH, ns), dim3(256), 0, s, hs, 0, part);
-  hipLaunchKernelGGL(k_hb_fold, dim3(nb_(ns, 64)), dim3(64), 0, s, hs, ns, part, 3, 1);
-  if (batched) {
-    launch_stencil_batch(B.plan[4][0], B.grid, s);
-  } else {
-    for (int i = s0; i < s1; i++) launch_stencil_batch(B.plan[4][1 + i], B.grid, s);
-  }
-  hipLaunchKernelGGL(k_hb_init, dim3(16, ns), dim3(256), 0, s, hs);
-  hipLaunchKernelGGL(k_hb_sum, dim3(HCH, ns), dim3(256), 0, s, hs, 1, part);
-  hipLaunchKernelGGL(k_hb_fold, dim3(nb_(ns, 64)), dim3(64), 0, s, hs, ns, part, 0, 0);
-  HIPCK(hipGetLastError());
-}
-
-void hartree_iter(Batch &B, int s0, int s1, bool batched, int ncgmin, int ncgmax, double eps,
-                  hipStream_t s) {
-  constexpr int ncgres = 801;  // restart period of parameters.inp
-  const int ns = s1 - s0;
-  HSys *hs = B.hs + s0;
-  double *part = B.hpart + (long)s0 * HCH;
-  hipLaunchKernelGGL(k_hb_begin, dim3(nb_(ns, 64)), dim3(64), 0, s, hs, ns, B.alldone);
+  hipLaunchKernelGGL(k_hb_fold, dim3(nb_(ns, 64)), dim3(64), 0, s, hs, ns, part, 1);
   if (batched) {
     launch_stencil_batch(B.plan[3][0], B.grid, s);
   } else {
     for (int i = s0; i < s1; i++) launch_stencil_batch(B.plan[3][1 + i], B.grid, s);
   }
-  hipLaunchKernelGGL(k_hb_pap, dim3(nb_(ns, 64)), dim3(64), 0, s, hs, ns);
-  hipLaunchKernelGGL(k_hb_update, dim3(HCH, ns), dim3(256), 0, s, hs, part);
-  hipLaunchKernelGGL(k_hb_r2r, dim3(nb_(ns, 64)), dim3(64), 0, s, hs, ns, part);
-  hipLaunchKernelGGL(k_hb_dir, dim3(16, ns), dim3(256), 0, s, hs, ncgres);
-  hipLaunchKernelGGL(k_hb_check, dim3(nb_(ns, 64)), dim3(64), 0, s, hs, ns, eps, ncgmin, ncgmax,
-                     B.alldone);
+  hipLaunchKernelGGL(k_hb_init, dim3(16, ns), dim3(256), 0, s, hs);
+  hipLaunchKernelGGL(k_hb_sum, dim3(HCH, ns), dim3(256), 0, s, hs, 1, part);
+  hipLaunchKernelGGL(k_hb_fold, dim3(nb_(ns, 64)), dim3(64), 0, s, hs, ns, part, 0);
   HIPCK(hipGetLastError());
 }
 
-int alldone(Batch &B, hipStream_t s) {
-  int h = 0;
-  HIPCK(hipMemcpyAsync(&h, B.alldone, sizeof(int), hipMemcpyDeviceToHost, s));
-  HIPCK(hipStreamSynchronize(s));
-  return h;
+// one iteration of systems [s0, s1), it = 0, 1, ...
+void hartree_iter(Batch &B, int s0, int s1, int it, hipStream_t s) {
+  hcg_iteration_batch(B.hcg_dev, B.hdir + B.hd0[s0], B.hd0[s1] - B.hd0[s0], B.hupd + B.hu0[s0], B.hu0[s1] - B.hu0[s0],
+                      B.hcg[0].tx, B.hcg[0].tz, it & 1, s);
 }
 
-void hartree_solve(Batch &B, int s0, int s1, bool batched, int ncgmax, double eps,
-                   hipStream_t s) {
+void hartree_solve(Batch &B, int s0, int s1, bool batched, int ncgmax, hipStream_t s) {
   hartree_start(B, s0, s1, batched, s);
-  const int blk = B.hart_blk;
-  for (int done = 0, it = 0; !done && it < ncgmax; it += blk) {
+  const int blk = B.hart_blk;  // even: a block starts with the same direction buffer
+  std::vector<int> st(3 * (s1 - s0));
+  // a solve that ends after ncgmax iterations is marked by the launch that follows them
+  for (int done = 0, it = 0; !done && it <= ncgmax; it += blk) {
     if (batched) {
       HIPCK(hipGraphLaunch(B.g_hart, s));
     } else {
-      for (int k = 0; k < blk; k++) hartree_iter(B, s0, s1, false, 1, ncgmax, eps, s);
+      for (int k = 0; k < blk; k++) hartree_iter(B, s0, s1, k, s);
     }
-    done = alldone(B, s);
+    HIPCK(hipMemcpyAsync(st.data(), B.hstate + 3 * s0, sizeof(int) * st.size(), hipMemcpyDeviceToHost, s));
+    HIPCK(hipStreamSynchronize(s));
+    done = 1;
+    for (size_t i = 0; i < st.size(); i += 3) done = done && st[i];
   }
+}
+
+// The iteration's rule of this step into the device table
+void hartree_rule(Batch &B, int ncgmax, double eps) {
+  if (B.hcg[0].ncgmax == ncgmax && B.hcg[0].eps == eps) return;
+  for (HcgArgs &a : B.hcg) {
+    a.ncgmax = ncgmax;
+    a.eps = eps;
+  }
+  HIPCK(hipMemcpy(B.hcg_dev, B.hcg.data(), sizeof(HcgArgs) * B.hcg.size(), hipMemcpyHostToDevice));
 }
 
 template <class F>
@@ -723,7 +649,10 @@ void prepare(Batch &B) {
   B.sval = B.alloc<double>(nbt);
   B.hs = B.alloc<HSys>(ns);
   B.hpart = B.alloc<double>((size_t)ns * HCH);
-  B.alldone = B.alloc<int>(1);
+  B.hsc = B.alloc<double>(3L * ns);
+  B.hstate = B.alloc<int>(3L * ns);
+  std::vector<int> st0(3L * ns, 0);
+  HIPCK(hipMemcpy(B.hstate, st0.data(), sizeof(int) * st0.size(), hipMemcpyHostToDevice));
   autotune(B, s);
   std::vector<BandRef> br(nbt);
   std::vector<HSys> hs(ns);
@@ -733,18 +662,49 @@ void prepare(Batch &B) {
     S.sparts = stencil_batch_parts(S.g, 4, S.M, B.P);
     S.nparts = S.sparts + expand_nparts(S.ctx->pl);
     S.part = S.alloc<double>((size_t)S.nparts * S.M);
-    S.hparts = stencil_batch_parts(S.g, 4, 1, B.P);
-    S.hpart = S.alloc<double>(S.hparts);
     for (int l = 0; l < S.M; l++) {
       BandRef &r = br[S.band0 + l];
       r.psi = S.psi + n * l; r.hpsi = S.hpsi + n * l; r.p = S.p + n * l; r.hp = S.hp + n * l;
       r.part = S.part + (long)S.nparts * l; r.n = n; r.nparts = (int)S.nparts; r.dv = S.g.dv();
     }
     HSys &H = hs[i];
-    H.rho = S.rho; H.vh = S.vh; H.b = S.hb; H.r = S.hr; H.p = S.hpv; H.ap = S.hap; H.avhs = S.havhs;
-    H.sc = S.hsc; H.part = S.hpart; H.state = S.hstate; H.n = n; H.np = (int)S.hparts;
-    H.dvo = 1.0 / (double)n;  // dV / Omega of the periodic cell
+    H.rho = S.rho; H.vh = S.vh; H.r = S.hr; H.p = S.hpv; H.ap = S.hap; H.sc = B.hsc + 3 * i;
+    H.state = B.hstate + 3 * i; H.n = n;
+    HcgArgs a{};
+    a.nx = S.g.nx; a.ny = S.g.ny; a.nz = S.g.nz; a.px = a.py = a.pz = 1;
+    double w[9];
+    fd_coefficients(4, w);
+    for (int m = 0; m < 9; m++) {
+      a.cx[m] = w[m] / S.g.dx / S.g.dx * (-0.5);
+      a.cy[m] = w[m] / S.g.dy / S.g.dy * (-0.5);
+      a.cz[m] = w[m] / S.g.dz / S.g.dz * (-0.5);
+    }
+    a.c0 = a.cx[0] + a.cy[0] + a.cz[0];
+    a.n = n; a.vh = S.vh; a.r = S.hr; a.p[0] = S.hpv; a.p[1] = S.hpw; a.ap = S.hap; a.rr = H.sc; a.state = H.state;
+    a.ncgres = 801;  // restart period of parameters.inp
+    a.ncgmin = 1;
+    a.dvo = 1.0 / (double)n;  // dV / Omega of the periodic cell
+    B.hcg.push_back(a);
   }
+  // the Hartree iteration's tiles, partial sums and units
+  hcg_plan_batch(B.hcg.data(), ns);
+  B.hd0.assign(1, 0);
+  B.hu0.assign(1, 0);
+  std::vector<int2> ud, uu;
+  for (int i = 0; i < ns; i++) {
+    HcgArgs &a = B.hcg[i];
+    a.part_p = B.alloc<double>(a.np);
+    a.part_r = B.alloc<double>(a.nr);
+    for (int k = 0; k < a.np; k++) ud.push_back(make_int2(i, k));
+    for (int k = 0; k < a.nr; k++) uu.push_back(make_int2(i, k));
+    B.hd0.push_back((int)ud.size());
+    B.hu0.push_back((int)uu.size());
+  }
+  B.hcg_dev = B.alloc<HcgArgs>(ns);
+  B.hdir = B.alloc<int2>(ud.size());
+  B.hupd = B.alloc<int2>(uu.size());
+  HIPCK(hipMemcpy(B.hdir, ud.data(), sizeof(int2) * ud.size(), hipMemcpyHostToDevice));
+  HIPCK(hipMemcpy(B.hupd, uu.data(), sizeof(int2) * uu.size(), hipMemcpyHostToDevice));
   HIPCK(hipMemcpy(B.bands, br.data(), sizeof(BandRef) * nbt, hipMemcpyHostToDevice));
   HIPCK(hipMemcpy(B.hs, hs.data(), sizeof(HSys) * ns, hipMemcpyHostToDevice));
   // orthonormalisation tables (param "batch_ortho", default 1, read once here)
@@ -837,13 +797,10 @@ int batch_add(void *h, int n, double hh, int nbands, int natom, int num_list, co
   S->ones = S->alloc<double>(nbands);
   S->rho = S->alloc<double>(N);
   S->vh = S->alloc<double>(N);
-  S->hb = S->alloc<double>(N);
   S->hr = S->alloc<double>(N);
   S->hpv = S->alloc<double>(N);
+  S->hpw = S->alloc<double>(N);
   S->hap = S->alloc<double>(N);
-  S->havhs = S->alloc<double>(N);
-  S->hsc = S->alloc<double>(8);
-  S->hstate = S->alloc<int>(2);
   auto up = [&](void *dst, const void *src, size_t bytes) {
     Arr a(src, bytes, Arr::In);
     HIPCK(hipMemcpyAsync(dst, a.v(), bytes, hipMemcpyDeviceToDevice, s));
@@ -876,20 +833,21 @@ void batch_step(void *h, int batched, int ncgmax, double epsvh) {
   prepare(*B);
   hipStream_t s = lib().stream;
   const int ns = (int)B->sys.size();
+  hartree_rule(*B, ncgmax, epsvh);
   if (batched) {
     Timed t("batch_step", 0.0);
     if (!B->g_band) B->g_band = capture(s, [&] { band_step(*B, 0, ns, true, s); });
     HIPCK(hipGraphLaunch(B->g_band, s));
     if (!B->g_hart)
       B->g_hart = capture(s, [&] {
-        for (int k = 0; k < B->hart_blk; k++) hartree_iter(*B, 0, ns, true, 1, ncgmax, epsvh, s);
+        for (int k = 0; k < B->hart_blk; k++) hartree_iter(*B, 0, ns, k, s);
       });
-    hartree_solve(*B, 0, ns, true, ncgmax, epsvh, s);
+    hartree_solve(*B, 0, ns, true, ncgmax, s);
   } else {
     Timed t("batch_loop", 0.0);
     for (int i = 0; i < ns; i++) {
       band_step(*B, i, i + 1, false, s);
-      hartree_solve(*B, i, i + 1, false, ncgmax, epsvh, s);
+      hartree_solve(*B, i, i + 1, false, ncgmax, s);
     }
   }
   sync();
@@ -924,10 +882,10 @@ void batch_get(void *h, int i, double *psi, double *sval, double *vh, int *iters
     a.finish();
   }
   if (iters) {
-    int st[2];
-    HIPCK(hipMemcpyAsync(st, S.hstate, sizeof(st), hipMemcpyDeviceToHost, s));
+    int st[3];
+    HIPCK(hipMemcpyAsync(st, B->hstate + 3 * i, sizeof(st), hipMemcpyDeviceToHost, s));
     sync();
-    *iters = st[1];
+    *iters = st[2];
   }
 }
 

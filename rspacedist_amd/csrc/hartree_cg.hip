@@ -11,6 +11,8 @@
 // Small grids are bound by the launches and the two folds of partial sums, 128^3 by the passes
 // (the update moves 100 MB in 16 us) and the tile halos.  Updating V one launch late, where its p
 // is read anyway (nine passes), was no faster: 39 us at 128^3, 17 at 64^3.
+// Twelve cells of 27^3 to 62^3 points in lock step (1.35 M points): 100 us with the stencil over a
+// list of plane tiles, an update, a direction and four small control launches, 30 us here.
 #include "hartree_cg.hpp"
 
 #include <algorithm>
@@ -37,15 +39,15 @@ __device__ inline double sum256(double s, double *red4) {  // valid in thread 0
   return ((red4[0] + red4[1]) + red4[2]) + red4[3];
 }
 
-// p = r + beta p, A p and the <p|A p> partials (zero from a work-group without a tile).  A work-group owns a tile of TX x (256 / TX)
-// columns and TZ planes; each thread loads its column's TZ + 2 NF values of r and p into
+// Work-group blk of nblk of one solve: p = r + beta p, A p and the <p|A p> partials (zero from a
+// work-group without a tile).  A work-group owns a tile of TX x (256 / TX) columns and TZ planes; each thread loads its column's TZ + 2 NF values of r and p into
 // registers and the work-group loads the tile's x and y halos, all in one batch of independent
 // loads that is in flight while <r|r> is folded; the new p then goes through LDS for the x and y
 // neighbours, with one barrier, and the z neighbours are in registers.  The tile has no serial
 // march, so a small grid's iteration is one memory latency long, and the tile's halos (2 x its
 // own points at 32 x 8 x 8) come from L2.
 template <int NF, int TX, int TZ>
-__global__ __launch_bounds__(256) void k_hcg_direction(HcgArgs a, int par) {
+__device__ inline void hcg_direction(const HcgArgs &a, int par, int blk, int nblk) {
   constexpr int TY = 256 / TX, W = TX + 2 * NF, WY = TY + 2 * NF, NZ = TZ + 2 * NF;
   constexpr int NXH = (2 * NF * TY * TZ + 255) / 256, NYH = (2 * NF * TX * TZ + 255) / 256;
   __shared__ double box[TZ][WY][W];
@@ -53,16 +55,18 @@ __global__ __launch_bounds__(256) void k_hcg_direction(HcgArgs a, int par) {
   if (a.state[0]) return;  // uniform: the solve has finished
   const int t = threadIdx.x, lx = t % TX, ly = t / TX;
   const int k = a.state[1];
-  const double *pold = a.p[par];
-  double *pnew = a.p[1 - par];
+  // (not a.p[par]: an indexed member would put a copied argument struct into scratch memory)
+  const double *pold = par ? a.p[1] : a.p[0];
+  double *pnew = par ? a.p[0] : a.p[1];
   const long plane = (long)a.nx * a.ny;
   const int ntile = a.ntx * a.nty * a.ntz;
   double beta = 0.0, dsum = 0.0;
   bool folded = false;
   // each XCD takes a contiguous eighth of the tiles, so most halos are read by the XCD whose L2
-  // holds them already (work-group g runs on XCD g mod 8; the grid is a multiple of 8)
-  const int per = (ntile + 7) / 8, xcd = blockIdx.x & 7, t1 = min(ntile, (xcd + 1) * per);
-  for (int tile = xcd * per + (blockIdx.x >> 3); tile < t1; tile += gridDim.x >> 3) {
+  // holds them already (work-group g runs on XCD g mod 8; nblk is a multiple of 8, and so is the grid index
+  // of the solve's first work-group)
+  const int per = (ntile + 7) / 8, xcd = blk & 7, t1 = min(ntile, (xcd + 1) * per);
+  for (int tile = xcd * per + (blk >> 3); tile < t1; tile += nblk >> 3) {
     const int x0 = tile % a.ntx * TX, y0 = tile / a.ntx % a.nty * TY, z0 = tile / (a.ntx * a.nty) * TZ;
     const int ex = min(TX, a.nx - x0), ey = min(TY, a.ny - y0), ez = min(TZ, a.nz - z0);
     const int x = x0 + lx, y = y0 + ly;
@@ -121,14 +125,14 @@ __global__ __launch_bounds__(256) void k_hcg_direction(HcgArgs a, int par) {
         const double r2r = fold256(a.part_r, a.nr, red);
         const int last = k - 1;
         if (last >= a.ncgmin && (last >= a.ncgmax || sqrt(r2r * a.dvo) <= a.eps)) {
-          if (blockIdx.x == 0 && t == 0) {
+          if (blk == 0 && t == 0) {
             a.state[2] = last;
             a.state[0] = 1;
           }
           return;
         }
         beta = last % a.ncgres == 0 ? 0.0 : r2r / a.rr[last & 1];
-        if (blockIdx.x == 0 && t == 0) a.rr[k & 1] = r2r;
+        if (blk == 0 && t == 0) a.rr[k & 1] = r2r;
       }
     } else {
       __syncthreads();  // the previous tile's values have been read
@@ -169,17 +173,28 @@ __global__ __launch_bounds__(256) void k_hcg_direction(HcgArgs a, int par) {
     }
   }
   const double tot = sum256(dsum, red);
-  if (t == 0) a.part_p[blockIdx.x] = tot;
+  if (t == 0) a.part_p[blk] = tot;
+}
+template <int NF, int TX, int TZ>
+__global__ __launch_bounds__(256) void k_hcg_direction(HcgArgs a, int par) {
+  hcg_direction<NF, TX, TZ>(a, par, blockIdx.x, gridDim.x);
+}
+// several solves in one launch: unit[g] = {solve, work-group of the solve}
+template <int NF, int TX, int TZ>
+__global__ __launch_bounds__(256) void k_hcg_direction_batch(const HcgArgs *tab, const int2 *unit, int par) {
+  const int2 u = unit[blockIdx.x];
+  const HcgArgs a = tab[u.x];
+  hcg_direction<NF, TX, TZ>(a, par, u.y, a.np);
 }
 
 // V += alpha p, r -= alpha A p and the <r|r> partials; the first batch of loads is in flight
 // while <p|A p> is folded
-__global__ __launch_bounds__(256) void k_hcg_update(HcgArgs a, int par) {
+__device__ inline void hcg_update(const HcgArgs &a, int par, int blk) {
   constexpr int P = 8;
   __shared__ double red[4];
   if (a.state[0]) return;
-  const double *p = a.p[1 - par];
-  const long i0 = blockIdx.x * a.chunk + threadIdx.x, i1 = min(a.n, (blockIdx.x + 1) * a.chunk);
+  const double *p = par ? a.p[0] : a.p[1];
+  const long i0 = blk * a.chunk + threadIdx.x, i1 = min(a.n, (blk + 1) * a.chunk);
   double v[P], q[P], r[P], w[P];
   auto load = [&](long i) {
 #pragma unroll
@@ -207,9 +222,15 @@ __global__ __launch_bounds__(256) void k_hcg_update(HcgArgs a, int par) {
   }
   s = sum256(s, red);
   if (threadIdx.x == 0) {
-    a.part_r[blockIdx.x] = s;
-    if (blockIdx.x == 0) a.state[1] += 1;
+    a.part_r[blk] = s;
+    if (blk == 0) a.state[1] += 1;
   }
+}
+__global__ __launch_bounds__(256) void k_hcg_update(HcgArgs a, int par) { hcg_update(a, par, blockIdx.x); }
+__global__ __launch_bounds__(256) void k_hcg_update_batch(const HcgArgs *tab, const int2 *unit, int par) {
+  const int2 u = unit[blockIdx.x];
+  const HcgArgs a = tab[u.x];
+  hcg_update(a, par, u.y);
 }
 
 template <int NF>
@@ -226,25 +247,61 @@ void direction(const HcgArgs &a, int par, hipStream_t s) {
   }
 }
 
+template <int TX, int TZ>
+void direction_batch(const HcgArgs *tab, const int2 *unit, int nblk, int par, hipStream_t s) {
+  hipLaunchKernelGGL((k_hcg_direction_batch<4, TX, TZ>), dim3(nblk), dim3(256), 0, s, tab, unit, par);
+}
+
+int up(int n, int t) { return (n + t - 1) / t; }
+// tiles and work-groups with tx x (256 / tx) x tz tiles, and points per update work-group
+void split(HcgArgs &a, int tx, int tz, long chunk) {
+  a.tx = tx;
+  a.tz = tz;
+  a.ntx = up(a.nx, tx);
+  a.nty = up(a.ny, 256 / tx);
+  a.ntz = up(a.nz, tz);
+  a.np = (int)std::min<long>(HCG_PARTS, ((long)a.ntx * a.nty * a.ntz + 7) / 8 * 8);
+  a.chunk = std::max(chunk, ((a.n + HCG_PARTS - 1) / HCG_PARTS + 255) / 256 * 256);
+  a.nr = (int)((a.n + a.chunk - 1) / a.chunk);
+}
+int planes(long tiles4) { return tiles4 < 1024 ? 2 : tiles4 <= 8192 ? 4 : 8; }
+
 }  // namespace
 
 void hcg_plan(HcgArgs &a, int nfh) {
-  auto up = [](int n, int t) { return (n + t - 1) / t; };
   // 32 x 8 columns where 16 x 16 would leave more of the tiles empty; the planes per tile by
   // the number of tiles: few tiles want the shortest launch (2 planes: 40^3 11.7 us per iteration
   // against 12.5 with 4 and 14.3 with 8), 128^3 fewer halo rows (4: 38.4 us, 2: 41.2, 8: 42.0),
   // and far past the chip's capacity the z halo costs most (256^3, 8: 328 us, 4: 351)
   const long c32 = (long)up(a.nx, 32) * up(a.ny, 8), c16 = (long)up(a.nx, 16) * up(a.ny, 16);
-  a.tx = c32 < c16 ? 32 : 16;
-  const long tiles4 = std::min(c16, c32) * up(a.nz, 4);
-  a.tz = tiles4 < 1024 ? 2 : tiles4 <= 8192 ? 4 : 8;
-  a.ntx = up(a.nx, a.tx);
-  a.nty = up(a.ny, 256 / a.tx);
-  a.ntz = up(a.nz, a.tz);
-  a.np = (int)std::min<long>(HCG_PARTS, ((long)a.ntx * a.nty * a.ntz + 7) / 8 * 8);
-  a.nr = (int)std::min<long>(HCG_PARTS, (a.n + 255) / 256);
-  a.chunk = ((a.n + a.nr - 1) / a.nr + 255) / 256 * 256;
-  a.nr = (int)((a.n + a.chunk - 1) / a.chunk);
+  split(a, c32 < c16 ? 32 : 16, planes(std::min(c16, c32) * up(a.nz, 4)), 256);
+}
+
+void hcg_plan_batch(HcgArgs *a, int ns) {
+  long t16 = 0, t32 = 0, n = 0;  // tiles of four planes, points
+  for (int i = 0; i < ns; i++) {
+    t16 += (long)up(a[i].nx, 16) * up(a[i].ny, 16) * up(a[i].nz, 4);
+    t32 += (long)up(a[i].nx, 32) * up(a[i].ny, 8) * up(a[i].nz, 4);
+    n += a[i].n;
+  }
+  const int tx = t32 < t16 ? 32 : 16, tz = planes(std::min(t16, t32));
+  const long chunk = std::min(2048L, std::max(256L, n / 1024 / 256 * 256));  // about 1024 work-groups
+  for (int i = 0; i < ns; i++) split(a[i], tx, tz, chunk);
+}
+
+void hcg_iteration_batch(const HcgArgs *dev, const int2 *dir_unit, int ndir, const int2 *upd_unit, int nupd, int tx,
+                         int tz, int parity, hipStream_t s) {
+  if (tx == 32) {
+    if (tz == 8) direction_batch<32, 8>(dev, dir_unit, ndir, parity, s);
+    else if (tz == 4) direction_batch<32, 4>(dev, dir_unit, ndir, parity, s);
+    else direction_batch<32, 2>(dev, dir_unit, ndir, parity, s);
+  } else {
+    if (tz == 8) direction_batch<16, 8>(dev, dir_unit, ndir, parity, s);
+    else if (tz == 4) direction_batch<16, 4>(dev, dir_unit, ndir, parity, s);
+    else direction_batch<16, 2>(dev, dir_unit, ndir, parity, s);
+  }
+  hipLaunchKernelGGL(k_hcg_update_batch, dim3(nupd), dim3(256), 0, s, dev, upd_unit, parity);
+  HIPCK(hipGetLastError());
 }
 
 void hcg_iteration(const HcgArgs &a, int nfh, int parity, hipStream_t s) {

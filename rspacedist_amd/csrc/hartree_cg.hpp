@@ -27,4 +27,11 @@ void hcg_plan(HcgArgs &a, int nfh);
 // written; p[0] must hold finite values before the first
 void hcg_iteration(const HcgArgs &a, int nfh, int parity, hipStream_t s);
 
+// Several solves with nfh = 4 in lock step: one tile shape for all of them, the arguments in a
+// device table and a table {solve, work-group of the solve} per launch, each solve's np (nr)
+// work-groups in order.  A range of solves may be run by itself with its part of the tables.
+void hcg_plan_batch(HcgArgs *a, int ns);
+void hcg_iteration_batch(const HcgArgs *dev, const int2 *dir_unit, int ndir, const int2 *upd_unit, int nupd, int tx,
+                         int tz, int parity, hipStream_t s);
+
 }  // namespace kukan

@@ -59,7 +59,6 @@ struct SP {
   const double *veff;
   double cx[9], cy[9], cz[9], c0;
   int accumulate;
-  const int *skip;
   const int *row_ptr;
   const int2 *ent;
   const double *vnl;
@@ -94,7 +93,6 @@ __device__ inline double val(const SP &p, const double *base, int x, int y, int 
 template <int NF>
 __global__ __launch_bounds__(256) void k_stencil(SP p) {
   __shared__ double red[4];
-  if (p.skip && *p.skip) return;  // uniform: a device-side loop has finished
   const int nxb = (p.nx + 63) / 64;
   const int x = (blockIdx.x % nxb) * 64 + threadIdx.x;
   const int y = blockIdx.y * 4 + threadIdx.y;
@@ -178,7 +176,6 @@ struct SL {
   const double *veff;
   double cx[9], cy[9], cz[9], c0;
   int accumulate;
-  const int *skip;
   const int *row_ptr;
   const int2 *ent;
   const double *vnl;
@@ -431,7 +428,6 @@ template <int NF, int P, int MODE>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(stencil_waves<NF, P, MODE>()))) void k_stencil_lds(SL p) {
   extern __shared__ double lds[];
   __shared__ double red[8];
-  if (p.skip && *p.skip) return;  // uniform: a device-side loop has finished
   const int L = blockIdx.x, xcd = L & 7, j = L >> 3;
   const int per = p.ntile * p.nzch;
   int b, rem;
@@ -460,7 +456,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NF <= 4 && 
   for (long it = blockIdx.x; it < total; it += gridDim.x) {
     while (s + 1 < nsys && start[s + 1] <= it) s++;  // items ascend, so s only moves forward
     const SL p = sl[s];
-    if (p.skip && *p.skip) continue;
     const long j = it - start[s];
     const int per = p.ntile * p.nzch;
     const int b = (int)(j / per), rem = (int)(j % per);
@@ -1332,7 +1327,6 @@ void launch_stencil(const StencilCall &c, hipStream_t s) {
   }
   p.c0 = p.cx[0] + p.cy[0] + p.cz[0];
   p.accumulate = c.accumulate ? 1 : 0;
-  p.skip = c.skip;
   if (c.pl && c.coef && c.pl->nent > 0) {
     if (c.coef_band_fastest != stencil_band_fastest_coef(g, c.halo_in))
       throw Error(1, "stencil: projector coefficients in the wrong layout");
@@ -1345,7 +1339,7 @@ void launch_stencil(const StencilCall &c, hipStream_t s) {
     q.nx = g.nx; q.ny = g.ny; q.nz = g.nz; q.px = p.px; q.py = p.py; q.pz = p.pz;
     q.in = c.in; q.ld_in = c.ld_in; q.out = c.out; q.ld_out = c.ld_out; q.veff = c.veff;
     for (int m = 0; m < 9; m++) { q.cx[m] = p.cx[m]; q.cy[m] = p.cy[m]; q.cz[m] = p.cz[m]; }
-    q.c0 = p.c0; q.accumulate = p.accumulate; q.skip = p.skip;
+    q.c0 = p.c0; q.accumulate = p.accumulate;
     q.row_ptr = p.row_ptr; q.ent = p.ent; q.vnl = p.vnl; q.coef = p.coef; q.ld_coef = p.ld_coef;
     q.num_list = p.num_list; q.nprjmx = p.nprjmx; q.iprj_slot = p.iprj_slot;
     q.dotp = c.dot_partial;
@@ -1423,7 +1417,7 @@ StencilBatchPlan plan_stencil_batch(const std::vector<StencilCall> &calls, bool 
     SL q{};
     q.nx = g.nx; q.ny = g.ny; q.nz = g.nz;
     q.px = g.nperi >= 1; q.py = g.nperi >= 2; q.pz = g.nperi >= 3;
-    q.in = c.in; q.ld_in = c.ld_in; q.out = c.out; q.ld_out = c.ld_out; q.skip = c.skip;
+    q.in = c.in; q.ld_in = c.ld_in; q.out = c.out; q.ld_out = c.ld_out;
     q.accumulate = c.accumulate ? 1 : 0;
     if (res) {
       q.in2 = c.in2; q.eps = c.eps; q.sign = c.sign;

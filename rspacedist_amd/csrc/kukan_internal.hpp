@@ -160,7 +160,6 @@ struct StencilCall {
   double *dot_partial = nullptr;     // optional: per-block partial sums of in_b . out_b
   long dot_ld = 0;                   // band stride of dot_partial (0: number of parts)
   int nfh_coeffs = 0;                // if > 0: use this FD order (Hartree), no veff
-  const int *skip = nullptr;         // device flag: the launch does nothing while *skip != 0
   // residual-preconditioner form (batched plans only): in = sign (in - eps_b in2)
   const double *in2 = nullptr, *eps = nullptr;
   double sign = 1.0;

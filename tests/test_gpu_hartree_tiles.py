@@ -56,3 +56,31 @@ def test_tiles(kk, dims, nperi, nfh):
     ref = np.einsum("abc,xa,yb,zc->xyz", np.where(live, c / np.where(live, d, 1.0), 0.0), *q, optimize=True)
     assert np.linalg.norm(v - ref) <= 1.01 * eps * np.sqrt(rho.size) / d[live].min()
     assert kk.get_param("hartree_iterations") < 3000
+
+
+def test_lock_step(kk):
+    """Cells of different edges advanced together, their rule changed from step to step (an
+    iteration count inside, at and past a block of 16): each against its own solve from the same
+    density and start.  CG iterates of a few tens of iterations agree to the rounding of their
+    recurrences, ~1e-15 of the potential an iteration."""
+    from rspacedist_amd import batch, synth
+    b = batch.Batch()
+    cells = []
+    for n, h, m in ((8, 0.4, 2), (33, 0.3, 3), (17, 0.35, 1), (50, 0.3, 4)):
+        s = synth.make_system(n, h, 2, m, seed=n)
+        q, _ = np.linalg.qr(synth.smooth_bands(synth.random_bands(s), n, h))
+        b.add(s, np.asfortranarray(q / np.sqrt(s.dv)))
+        cells.append([s, np.zeros(s.npts)])
+    z = np.zeros(1)
+    for batched, ncgmax in ((True, 1), (True, 16), (False, 17), (True, 33), (False, 1), (True, 15)):
+        b.step(batched=batched, ncgmax=ncgmax, epsvh=1e-30)
+        for i, (s, start) in enumerate(cells):
+            psi, _, vh, its = b.get(i)
+            ref = start.copy()
+            kk.call("scf_hartree", nd=1, ncpx_d=s.n, ncpy_d=s.n, ncpz_d=s.n, nfh=4, ndisp=6, nperi=3, ncgres=801,
+                    ncgmin=1, ncgmax=ncgmax, xmax=s.xmax, ymax=s.xmax, zmax=s.xmax, epsvh=1e-30,
+                    rho_aug_dense=(psi ** 2).sum(axis=1), boundx=z, boundy=z, boundz=z, vh_dense=ref)
+            assert its == ncgmax
+            np.testing.assert_allclose(vh, ref, rtol=0, atol=1e-11 * np.abs(ref).max())
+            cells[i][1] = vh.copy()
+    b.close()
