@@ -212,125 +212,216 @@ inline unsigned nb_(long n, int t) { return (unsigned)((n + t - 1) / t); }
 // Psi <- Psi R^-1, the same Q as the reference's Gram-Schmidt (orthogonalization8f.F90:93-376)
 // in exact arithmetic.  The work of all systems runs in one launch per kernel over unit
 // tables (system-major), so loop mode launches the same kernels on one system's units.
-constexpr int GT = 32;          // band tile of the Gram partials
-constexpr long GCH = 16384;     // points per Gram work-group
-constexpr int OMAX = 128;       // bands per system (the Cholesky runs in 128 KB of LDS)
+// The products run on the FP64 matrix cores straight from global memory; the sizes (at most 128
+// bands) let a wave hold what a general product would stage.  12 cells of 27^3 to 62^3 points, 16
+// to 126 bands: Gram 2.44 -> 0.53 ms, factor and inverse 1.18 -> 0.16 ms, apply 2.14 -> 0.47 ms
+// (vector FMAs from LDS tiles, and a column of the inverse per thread, before).
+constexpr int OMAX = 128;  // bands per system (the Cholesky runs in 128 KB of LDS)
+constexpr int ONT = OMAX / 16;
+typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d4u __attribute__((ext_vector_type(4), aligned(8)));
 struct OSys {
   double *psi;
-  long n;
-  int M, ntile, nchunk, ntp;
+  long n, kc;  // points; points per Gram unit
+  int M, nt, nchunk;
   double dv;
-  double *G, *Rinv, *part;  // M x M, M x M, [tile pair][chunk][GT x GT]
+  double *G, *Rinv, *part;  // M x M, M x M (and 16 zeros), [pair of 16-band tiles][chunk][256]
   int *flag;                // 1: a pivot was not positive
 };
-struct GUnit {
-  int sys, tp, ti, tj, chunk;
+struct GUnit {  // Gram: points [item kc, ...) and which part of the pairs; reduction: pair of tiles
+  int sys, item, part;
 };
 struct AUnit {
   int sys;
-  long p0;  // first point of the 64-point tile
+  long p0;  // first point of the 128-point tile
 };
 
-// Gram partial of band tiles (ti, tj) over one chunk of points: 4 outputs per thread
-__global__ __launch_bounds__(256) void k_bgram_part(const OSys *os, const GUnit *units) {
-  __shared__ double A[GT][65], Bt[GT][65];
+// One wave: the upper tile pairs i <= j, J0 <= j < NT, of X^T X over points [k0, k1), all of them
+// in registers (NT = 6: 21 x 4 doubles per lane), so every value is loaded once, 32 bytes per lane,
+// and one 16-point step of loads is in flight while the products of the last run.  More than six
+// tiles do not fit 512 registers: their last one or two columns of pairs are a wave's work of
+// their own.  A lane's operand is the same for both sides: band l % 16 of its tile, points
+// 4 (l / 16) + s at step s.
+template <int NT, int J0>
+__device__ inline void gram_unit(const OSys &S, long k0, long k1, int chunk) {
+  const int lane = threadIdx.x, q = lane >> 4, c16 = lane & 15;
+  const double *col[NT];
+#pragma unroll
+  for (int f = 0; f < NT; f++)  // bands past the last repeat it (results unused)
+    col[f] = S.psi + S.n * min(16 * f + c16, S.M - 1) + k0 + 4 * q;
+  constexpr int PR0 = J0 * (J0 + 1) / 2, NP = NT * (NT + 1) / 2 - PR0;
+  d4 acc[NP];
+#pragma unroll
+  for (int i = 0; i < NP; i++) acc[i] = d4{0.0, 0.0, 0.0, 0.0};
+  auto mac = [&](const d4u *x) {
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+      int pr = 0;
+#pragma unroll
+      for (int j = J0; j < NT; j++)
+#pragma unroll
+        for (int i = 0; i <= j; i++, pr++)
+          acc[pr] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i][s], x[j][s], acc[pr], 0, 0, 0);
+    }
+  };
+  const long nf = (k1 - k0) / 16;
+  d4u x[NT], xn[NT];
+  if (nf > 0) {
+#pragma unroll
+    for (int f = 0; f < NT; f++) x[f] = *(const d4u *)col[f];
+    for (long st = 1; st < nf; st++) {
+#pragma unroll
+      for (int f = 0; f < NT; f++) xn[f] = *(const d4u *)(col[f] + 16 * st);
+      mac(x);
+#pragma unroll
+      for (int f = 0; f < NT; f++) x[f] = xn[f];
+    }
+    mac(x);
+  }
+  const int rem = (int)(k1 - k0 - 16 * nf);
+  if (rem > 0) {  // the last, partial step: points past k1 are zero
+#pragma unroll
+    for (int f = 0; f < NT; f++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) x[f][s] = 4 * q + s < rem ? col[f][16 * nf + s] : 0.0;
+    mac(x);
+  }
+#pragma unroll
+  for (int pr = 0; pr < NP; pr++) {
+    double *o = S.part + ((long)(PR0 + pr) * S.nchunk + chunk) * 256 + lane;
+#pragma unroll
+    for (int r = 0; r < 4; r++) o[64 * r] = acc[pr][r];
+  }
+}
+__global__ __launch_bounds__(64, 1) void k_bgram_part(const OSys *os, const GUnit *units) {
   const GUnit u = units[blockIdx.x];
   const OSys S = os[u.sys];
-  const long c0 = (long)u.chunk * GCH, c1 = min(S.n, c0 + GCH);
-  const int t = threadIdx.x, i = t & 31, j0 = t >> 5;
-  double acc[4] = {0.0, 0.0, 0.0, 0.0};
-  for (long p0 = c0; p0 < c1; p0 += 64) {
-    for (int e = t; e < GT * 64; e += 256) {
-      const int b = e >> 6, q = e & 63;
-      const long pt = p0 + q;
-      const int ba = u.ti * GT + b, bb = u.tj * GT + b;
-      A[b][q] = (ba < S.M && pt < c1) ? S.psi[(long)ba * S.n + pt] : 0.0;
-      Bt[b][q] = (bb < S.M && pt < c1) ? S.psi[(long)bb * S.n + pt] : 0.0;
-    }
-    __syncthreads();
-    for (int q = 0; q < 64; q++) {
-      const double a = A[i][q];
-#pragma unroll
-      for (int k = 0; k < 4; k++) acc[k] += a * Bt[j0 + 8 * k][q];
-    }
-    __syncthreads();
+  const long k0 = u.item * S.kc, k1 = min(S.n, k0 + S.kc);
+  switch (S.nt) {
+    case 1: gram_unit<1, 0>(S, k0, k1, u.item); break;
+    case 2: gram_unit<2, 0>(S, k0, k1, u.item); break;
+    case 3: gram_unit<3, 0>(S, k0, k1, u.item); break;
+    case 4: gram_unit<4, 0>(S, k0, k1, u.item); break;
+    case 5: gram_unit<5, 0>(S, k0, k1, u.item); break;
+    case 6: gram_unit<6, 0>(S, k0, k1, u.item); break;
+    default:
+      if (u.part == 0) gram_unit<6, 0>(S, k0, k1, u.item);
+      else if (S.nt == 7) gram_unit<7, 6>(S, k0, k1, u.item);
+      else gram_unit<8, 6>(S, k0, k1, u.item);
   }
-  double *o = S.part + ((long)u.tp * S.nchunk + u.chunk) * (GT * GT);
-#pragma unroll
-  for (int k = 0; k < 4; k++) o[i + GT * (j0 + 8 * k)] = acc[k];
 }
 
-// G tile (ti, tj) = dV sum over chunks in order
+// G tile pair = dV sum over chunks in order; register r of lane l is row l / 16 + 4 r, column l % 16
 __global__ __launch_bounds__(256) void k_bgram_reduce(const OSys *os, const GUnit *units) {
-  const GUnit u = units[blockIdx.x];  // chunk field unused: one unit per tile pair
+  const GUnit u = units[blockIdx.x];
   const OSys S = os[u.sys];
-  for (int e = threadIdx.x; e < GT * GT; e += 256) {
-    const int i = e % GT, j = e / GT, gi = u.ti * GT + i, gj = u.tj * GT + j;
-    double s = 0.0;
-    for (int c = 0; c < S.nchunk; c++) s += S.part[((long)u.tp * S.nchunk + c) * (GT * GT) + e];
-    if (gi < S.M && gj < S.M) S.G[gi + (long)S.M * gj] = S.dv * s;
-  }
+  int tj = 0, ti = u.item;
+  while (ti > tj) ti -= ++tj;
+  const int t = threadIdx.x, lane = t & 63;
+  const int gi = 16 * ti + (lane >> 4) + 4 * (t >> 6), gj = 16 * tj + (lane & 15);
+  const double *p = S.part + (long)u.item * S.nchunk * 256 + t;
+  double s = 0.0;
+#pragma unroll 8
+  for (int c = 0; c < S.nchunk; c++) s += p[256L * c];
+  if (gi < S.M && gj < S.M) S.G[gi + (long)S.M * gj] = S.dv * s;
 }
 
-// upper Cholesky factor of G in LDS, then its inverse (one column per thread), per system
-__global__ __launch_bounds__(256) void k_bchol_inv(const OSys *os) {
-  __shared__ double R[OMAX * OMAX];
+// R^-1 of G = R^T R per system in LDS, by eliminating [G | 1]: the upper triangle holds what is
+// left of G, the strictly lower one the rows of R^-T found so far.  Step k divides row k of both
+// by its pivot's root (w) and subtracts w_i w_j from every row i > k; its work does not shrink
+// with k, and no thread waits on a chain longer than a step.
+__global__ __launch_bounds__(1024) void k_bchol_inv(const OSys *os) {
+  __shared__ double A[OMAX * OMAX], w[2][OMAX], dinv[OMAX];
   __shared__ int bad;
   const OSys S = os[blockIdx.x];
-  const int M = S.M, t = threadIdx.x;
-  for (int e = t; e < M * M; e += 256) R[e] = S.G[e];
+  const int M = S.M, t = threadIdx.x, tx = t & 31, ty = t >> 5;
+  for (int j = ty; j < M; j += 32)
+    for (int i = tx; i < M; i += 32) A[i + M * j] = i <= j ? S.G[i + (long)M * j] : 0.0;
   if (t == 0) bad = 0;
   __syncthreads();
   for (int k = 0; k < M; k++) {
-    if (t == 0) {
-      const double d = R[k + M * k];
-      if (!(d > 0.0)) bad = 1;
-      R[k + M * k] = d > 0.0 ? sqrt(d) : 1.0;
+    double *wk = w[k & 1];
+    if (t < M) {
+      const double d = A[k + M * k], f = 1.0 / (d > 0.0 ? sqrt(d) : 1.0);
+      if (t == k) {
+        if (!(d > 0.0)) bad = 1;
+        wk[t] = dinv[t] = f;
+      } else {
+        const double v = A[k + M * t] * f;
+        wk[t] = v;
+        if (t < k) A[k + M * t] = v;  // row k of R^-T
+      }
     }
     __syncthreads();
-    const double rkk = R[k + M * k];
-    for (int j = k + 1 + t; j < M; j += 256) R[k + M * j] /= rkk;
-    __syncthreads();
-    const int m = M - k - 1;  // the trailing upper triangle, (i, j) with k < i <= j
-    for (int e = t; e < m * m; e += 256) {
-      const int i = k + 1 + e % m, j = k + 1 + e / m;
-      if (i <= j) R[i + M * j] -= R[k + M * i] * R[k + M * j];
+    for (int j = ty; j < M; j += 32) {
+      const double wj = wk[j];
+      const int i0 = k + 1, i1 = j <= k ? M : j + 1;  // rows of R^-T, or the rows of G above j
+      for (int i = i0 + tx; i < i1; i += 32) A[i + M * j] -= wk[i] * wj;
     }
     __syncthreads();
   }
-  // X = R^-1 (upper): column j by back substitution, written to Rinv (zero below the diagonal)
-  for (int j = t; j < M; j += 256) {
-    double *X = S.Rinv + (long)M * j;
-    for (int i = j + 1; i < M; i++) X[i] = 0.0;
-    X[j] = 1.0 / R[j + M * j];
-    for (int i = j - 1; i >= 0; i--) {
-      double s = 0.0;
-      for (int k = i + 1; k <= j; k++) s += R[i + M * k] * X[k];
-      X[i] = -s / R[i + M * i];
-    }
-  }
+  for (int j = ty; j < M; j += 32)
+    for (int i = tx; i < M; i += 32) S.Rinv[i + (long)M * j] = i < j ? A[j + M * i] : i == j ? dinv[i] : 0.0;
   if (t == 0) *S.flag = bad;
 }
 
-// Psi <- Psi R^-1 on a tile of 64 points: the tile's bands staged in LDS, in place
+// Psi <- Psi R^-1, a wave per 32 points: it loads all its bands (8 NT doubles per lane), then
+// forms the rows of R^-T Psi^T tile by tile, so the update is in place without LDS.  Psi is the
+// right operand (and the result's columns): loads and stores are 16 consecutive points each, and
+// R^-1 (at most 128 KB) comes from the caches.
+template <int NT>
+__device__ inline void apply_unit(const OSys &S, long p0) {
+  const int lane = threadIdx.x & 63, q = lane >> 4, c16 = lane & 15;
+  double x[2][NT][4];
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+    const long pt = min(p0 + 16 * h + c16, S.n - 1);
+#pragma unroll
+    for (int f = 0; f < NT; f++)
+#pragma unroll
+      for (int s = 0; s < 4; s++) {
+        const int b = 16 * f + 4 * q + s;
+        x[h][f][s] = b < S.M ? S.psi[S.n * b + pt] : 0.0;
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < NT; j++) {
+    const double *rc = S.Rinv + (long)S.M * min(16 * j + c16, S.M - 1) + 4 * q;
+    d4 acc[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
+#pragma unroll
+    for (int f = 0; f <= j; f++) {
+      const d4u a = *(const d4u *)(rc + 16 * f);  // past the last band: zero bands in x
+#pragma unroll
+      for (int s = 0; s < 4; s++)
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+          acc[h] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s], x[h][f][s], acc[h], 0, 0, 0);
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const long pt = p0 + 16 * h + c16;
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const int b = 16 * j + q + 4 * r;
+        if (b < S.M && pt < S.n) S.psi[S.n * b + pt] = acc[h][r];
+      }
+    }
+  }
+}
 __global__ __launch_bounds__(256) void k_bortho_apply(const OSys *os, const AUnit *units) {
-  __shared__ double X[OMAX][64];
   const AUnit u = units[blockIdx.x];
   const OSys S = os[u.sys];
-  const int t = threadIdx.x, q = t & 63;
-  const long pt = u.p0 + q;
-  for (int e = t; e < S.M * 64; e += 256) {
-    const int b = e >> 6, qq = e & 63;
-    const long p = u.p0 + qq;
-    X[b][qq] = p < S.n ? S.psi[(long)b * S.n + p] : 0.0;
-  }
-  __syncthreads();
-  if (pt >= S.n) return;
-  for (int j = t >> 6; j < S.M; j += 4) {
-    const double *rc = S.Rinv + (long)S.M * j;
-    double y = 0.0;
-    for (int i = 0; i <= j; i++) y += X[i][q] * rc[i];
-    S.psi[(long)j * S.n + pt] = y;
+  const long p0 = u.p0 + 32 * (threadIdx.x >> 6);
+  if (p0 >= S.n) return;
+  switch (S.nt) {
+    case 1: apply_unit<1>(S, p0); break;
+    case 2: apply_unit<2>(S, p0); break;
+    case 3: apply_unit<3>(S, p0); break;
+    case 4: apply_unit<4>(S, p0); break;
+    case 5: apply_unit<5>(S, p0); break;
+    case 6: apply_unit<6>(S, p0); break;
+    case 7: apply_unit<7>(S, p0); break;
+    default: apply_unit<8>(S, p0); break;
   }
 }
 
@@ -501,9 +592,9 @@ void band_step(Batch &B, int s0, int s1, bool batched, hipStream_t s) {
   // Cholesky-QR of each system's bands
   if (B.ortho) {
     const int ng = B.g0[s1] - B.g0[s0], nr = B.r0[s1] - B.r0[s0], na = B.a0[s1] - B.a0[s0];
-    if (ng > 0) hipLaunchKernelGGL(k_bgram_part, dim3(ng), dim3(256), 0, s, B.osys, B.gunits + B.g0[s0]);
+    if (ng > 0) hipLaunchKernelGGL(k_bgram_part, dim3(ng), dim3(64), 0, s, B.osys, B.gunits + B.g0[s0]);
     if (nr > 0) hipLaunchKernelGGL(k_bgram_reduce, dim3(nr), dim3(256), 0, s, B.osys, B.runits + B.r0[s0]);
-    hipLaunchKernelGGL(k_bchol_inv, dim3(s1 - s0), dim3(256), 0, s, B.osys + s0);
+    hipLaunchKernelGGL(k_bchol_inv, dim3(s1 - s0), dim3(1024), 0, s, B.osys + s0);
     if (na > 0) hipLaunchKernelGGL(k_bortho_apply, dim3(na), dim3(256), 0, s, B.osys, B.aunits + B.a0[s0]);
   }
   HIPCK(hipGetLastError());
@@ -714,6 +805,11 @@ void prepare(Batch &B) {
     std::vector<GUnit> gu, ru;
     std::vector<AUnit> au;
     B.oflag = B.alloc<int>(ns);
+    long points = 0;
+    for (auto &sp : B.sys) points += sp->g.n();
+    // points per Gram wave: about one wave per SIMD of the chip, and no shorter than the
+    // partial sums it leaves are worth
+    const long kc = std::min(8192L, std::max(512L, points / 1024 / 16 * 16));
     B.g0.assign(1, 0);
     B.r0.assign(1, 0);
     B.a0.assign(1, 0);
@@ -724,21 +820,20 @@ void prepare(Batch &B) {
       o.psi = S.psi;
       o.n = S.g.n();
       o.M = S.M;
-      o.ntile = (S.M + GT - 1) / GT;
-      o.nchunk = (int)((o.n + GCH - 1) / GCH);
-      o.ntp = o.ntile * (o.ntile + 1) / 2;
+      o.nt = (S.M + 15) / 16;
+      o.kc = kc;
+      o.nchunk = (int)((o.n + kc - 1) / kc);
+      const int ntp = o.nt * (o.nt + 1) / 2;
       o.dv = S.g.dv();
       o.G = S.alloc<double>((size_t)S.M * S.M);
-      o.Rinv = S.alloc<double>((size_t)S.M * S.M);
-      o.part = S.alloc<double>((size_t)o.ntp * o.nchunk * GT * GT);
+      o.Rinv = S.alloc<double>((size_t)S.M * S.M + 16);
+      launch_fill(16, 0.0, o.Rinv + (size_t)S.M * S.M, s);
+      o.part = S.alloc<double>((size_t)ntp * o.nchunk * 256);
       o.flag = B.oflag + i;
-      int tp = 0;
-      for (int tj = 0; tj < o.ntile; tj++)
-        for (int ti = 0; ti <= tj; ti++, tp++) {
-          for (int c = 0; c < o.nchunk; c++) gu.push_back({i, tp, ti, tj, c});
-          ru.push_back({i, tp, ti, tj, 0});
-        }
-      for (long p0 = 0; p0 < o.n; p0 += 64) au.push_back({i, p0});
+      for (int c = 0; c < o.nchunk; c++)
+        for (int part = 0; part < (o.nt > 6 ? 2 : 1); part++) gu.push_back({i, c, part});
+      for (int tp = 0; tp < ntp; tp++) ru.push_back({i, tp, 0});
+      for (long p0 = 0; p0 < o.n; p0 += 128) au.push_back({i, p0});
       B.g0.push_back((int)gu.size());
       B.r0.push_back((int)ru.size());
       B.a0.push_back((int)au.size());

@@ -98,6 +98,31 @@ def test_batched_equals_loop_bitwise(kk):
     print(f"tuned tile P={kk.get_param('batch_tile_p'):.0f}, grid={kk.get_param('batch_grid'):.0f}")
 
 
+def test_orthonormalisation_tile_edges(kk):
+    """Band counts at the edges of the Gram's 16-band tiles (and of its six-tile waves) and grids
+    whose points end inside a step, a chunk and a 32-point tile, against the Cholesky-QR of the same
+    step's bands left as the update made them.  Bar: both Gram sums carry n eps of rounding, the
+    factor M eps, times the bands' condition squared (< 10 here): < 1e-12 of the largest entry."""
+    shapes = [(8, 1), (8, 128), (9, 15), (9, 16), (9, 17), (11, 33), (12, 96), (13, 97), (10, 112), (17, 113),
+              (15, 127), (29, 48)]
+    out = []
+    for ortho in (0, 1):
+        kk.set_param("batch_ortho", ortho)
+        systems = []
+        for n, m in shapes:
+            s = synth.make_system(n, 0.35, 2, m, seed=100 * n + m)
+            q, _ = np.linalg.qr(synth.random_bands(s))
+            systems.append((s, np.asfortranarray(q / np.sqrt(s.dv))))
+        b = _batch(systems)
+        b.step(batched=bool(ortho), ncgmax=1)
+        out.append([b.get(i)[0] for i in range(len(shapes))])
+        b.close()
+    for (s, _), raw, got in zip(systems, *out):
+        ref = np.linalg.solve(np.linalg.cholesky(s.dv * raw.T @ raw), raw.T).T
+        np.testing.assert_allclose(got, ref, rtol=0, atol=1e-12 * np.abs(ref).max())
+        assert np.abs(s.dv * got.T @ got - np.eye(s.nbands)).max() < 1e-12
+
+
 def test_batching_config_48_systems(kk):
     """The 48-system configuration (sizes in {32,48,64,80}^3, 16..128 bands, 2..24 atoms):
     batched (persistent stencil launches + graph replays) vs the per-system launch loop, same
