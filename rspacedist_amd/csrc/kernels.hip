@@ -199,10 +199,10 @@ struct SL {
 // point's z-column live in registers; plane z (TY rows plus NF halo rows on either side, each
 // row padded by NF wrapped or zero columns) is staged in LDS, so every x and y neighbour is an
 // unconditional LDS read.  Loads of plane z + NF + 1, of plane z + 1's halo rows and of
-// V_eff(z + 1) are issued before plane z is computed (one plane of prefetch), and the barriers
-// wait only for LDS, so HBM latency overlaps the arithmetic.
+// V_eff(z + 1) are issued before plane z is computed (one plane of prefetch, or two: D), and the
+// barriers wait only for LDS, so HBM latency overlaps the arithmetic.
 // One work-group's share: band b, y-tile `tile`, z-range `zch` (all arguments uniform).
-template <int NF, int P, int MODE>
+template <int NF, int P, int MODE, int D, int NT>
 __device__ inline void stencil_block(const SL &p, int b, int tile, int zch, double *lds,
                                      double *red) {
   constexpr bool RES = MODE == 1, COMB = MODE == 2 || MODE == 5, SYM = MODE == 5, UPD = MODE == 6;
@@ -210,7 +210,7 @@ __device__ inline void stencil_block(const SL &p, int b, int tile, int zch, doub
   // MODE 3: plain, also the partials of <c|c> (no max); MODE 4: plain, also the maxima of |c|
   // and |out| (no partials) - each keeps the plain kernel's accumulator count
   constexpr bool NORMS = MODE == 3, MAXES = MODE == 4;
-  constexpr int H = NF;  // halo values per thread: 2 NF rows x nx <= 512 NF for nx <= 256
+  constexpr int H = (2 * NF * 256 + NT - 1) / NT;  // halo values per thread: 2 NF rows of nx <= 256
   const int nx = p.nx, ny = p.ny, nz = p.nz, TY = p.TY, W = nx + 2 * NF;
   const long plane = (long)nx * ny;
   const int per = p.ntile * p.nzch;
@@ -259,7 +259,7 @@ __device__ inline void stencil_block(const SL &p, int b, int tile, int zch, doub
   int xq[P];
 #pragma unroll
   for (int q = 0; q < P; q++) {
-    const int idx = t + 512 * q;
+    const int idx = t + NT * q;
     const bool in_tile = idx < nx * TY;
     const int x = in_tile ? idx % nx : 0, yl = in_tile ? idx / nx : 0;
     const int gy = y0 + yl, gw = wrap_y(gy);
@@ -269,12 +269,12 @@ __device__ inline void stencil_block(const SL &p, int b, int tile, int zch, doub
     oxy[q] = x + nx * (gw < 0 ? 0 : gw);
     lcol[q] = (NF + yl) * W + NF + x;
   }
-  // halo rows: index i = t + 512 h over 2 NF rows x nx
+  // halo rows: index i = t + NT h over 2 NF rows x nx
   int hxy[H], hcol[H], hx[H];
   bool hv_ok[H];
 #pragma unroll
   for (int h = 0; h < H; h++) {
-    const int i = t + 512 * h;
+    const int i = t + NT * h;
     const bool ok = i < 2 * NF * nx;
     const int r = ok ? i / nx : 0, x = ok ? i % nx : 0;
     const int row = r < NF ? r : TY + r;
@@ -286,7 +286,7 @@ __device__ inline void stencil_block(const SL &p, int b, int tile, int zch, doub
   }
   // pad columns are zero for a non-periodic x axis and never rewritten
   if (!p.px)
-    for (int i = t; i < (TY + 2 * NF) * 2 * NF; i += 512) {
+    for (int i = t; i < (TY + 2 * NF) * 2 * NF; i += NT) {
       const int row = i / (2 * NF), c = i % (2 * NF);
       lds[row * W + (c < NF ? c : nx + c)] = 0.0;
     }
@@ -317,49 +317,55 @@ __device__ inline void stencil_block(const SL &p, int b, int tile, int zch, doub
   }
   // MODE 2: the second band and its H at the centre, prefetched like V_eff
   constexpr int YP = COMB ? P : 1;
-  double yf[YP], hf[YP];
-  double nxt[P], hvv[H], vf[P];
-  auto prefetch = [&](int z) {
+  // D planes of loads are in flight, a set of registers each
+  double yf[D][YP], hf[D][YP];
+  double nxt[D][P], hvv[D][H], vf[D][P];
+  auto prefetch = [&](int z, auto set) {
+    constexpr int S = decltype(set)::value;
     const long zn = zoff(z + NF), zh = (long)z * plane;
 #pragma unroll
     for (int q = 0; q < P; q++) {
       if (UPD) {
-        nxt[q] = (lv[q] && zn >= 0) ? ld3(zn + oxy[q], xnx[q], unx[q]) : 0.0;
+        nxt[S][q] = (lv[q] && zn >= 0) ? ld3(zn + oxy[q], xnx[q], unx[q]) : 0.0;
         if (!(lv[q] && zn >= 0)) xnx[q] = unx[q] = 0.0;
       } else {
-        nxt[q] = (lv[q] && zn >= 0) ? ld(zn + oxy[q]) : 0.0;
+        nxt[S][q] = (lv[q] && zn >= 0) ? ld(zn + oxy[q]) : 0.0;
       }
-      if (COMB && !SYM) yf[q] = sv[q] ? in2[zh + oxy[q]] : 0.0;
-      if (COMB) hf[q] = sv[q] ? hin[zh + oxy[q]] : 0.0;
-      vf[q] = (p.veff && sv[q]) ? p.veff[zh + oxy[q]] : 0.0;
+      if (COMB && !SYM) yf[S][q] = sv[q] ? in2[zh + oxy[q]] : 0.0;
+      if (COMB) hf[S][q] = sv[q] ? hin[zh + oxy[q]] : 0.0;
+      vf[S][q] = (p.veff && sv[q]) ? p.veff[zh + oxy[q]] : 0.0;
     }
 #pragma unroll
-    for (int h = 0; h < H; h++) hvv[h] = hv_ok[h] ? ld(zh + hxy[h]) : 0.0;
+    for (int h = 0; h < H; h++) hvv[S][h] = hv_ok[h] ? ld(zh + hxy[h]) : 0.0;
   };
-  prefetch(z0);
+  using set0 = std::integral_constant<int, 0>;
+  using set1 = std::integral_constant<int, D - 1>;
+  prefetch(z0, set0());
+  if (D == 2 && z0 + 1 < z1) prefetch(z0 + 1, set1());
   double dsum = 0.0, dsum2 = 0.0, dsum3 = 0.0, amax = 0.0, cmx = 0.0;
-  for (int z = z0; z < z1; z++) {
+  auto step = [&](int z, auto set) {
+    constexpr int S = decltype(set)::value;
     double vcur[P], ycur[YP], hcur[YP], xcen[UP], ucen[UP];
 #pragma unroll
     for (int q = 0; q < P; q++) {
 #pragma unroll
       for (int m = 0; m < 2 * NF; m++) col[q][m] = col[q][m + 1];
-      col[q][2 * NF] = nxt[q];
+      col[q][2 * NF] = nxt[S][q];
       if (UPD) {  // radius 1: the plane just prefetched is the next centre
         xcen[q] = xd[q];
         ucen[q] = ud[q];
         xd[q] = xnx[q];
         ud[q] = unx[q];
       }
-      if (COMB && !SYM) ycur[q] = yf[q];
-      if (COMB) hcur[q] = hf[q];
-      vcur[q] = vf[q];
-      if (t + 512 * q < nx * TY) put(lcol[q], xq[q], col[q][NF]);
+      if (COMB && !SYM) ycur[q] = yf[S][q];
+      if (COMB) hcur[q] = hf[S][q];
+      vcur[q] = vf[S][q];
+      if (t + NT * q < nx * TY) put(lcol[q], xq[q], col[q][NF]);
     }
 #pragma unroll
     for (int h = 0; h < H; h++)
-      if (hcol[h] >= 0) put(hcol[h], hx[h], hvv[h]);
-    if (z + 1 < z1) prefetch(z + 1);
+      if (hcol[h] >= 0) put(hcol[h], hx[h], hvv[S][h]);
+    if (z + D < z1) prefetch(z + D, set);
     __syncthreads();
     const long zh = (long)z * plane;
 #pragma unroll
@@ -392,31 +398,39 @@ __device__ inline void stencil_block(const SL &p, int b, int tile, int zch, doub
       }
     }
     __syncthreads();
+  };
+  if (D == 1) {
+    for (int z = z0; z < z1; z++) step(z, set0());
+  } else {
+    for (int z = z0; z < z1; z += 2) {
+      step(z, set0());
+      if (z + 1 < z1) step(z + 1, set1());
+    }
   }
   if (!MAXES && p.dotp) {
-    const double tot = block_sum<512>(dsum, red);
+    const double tot = block_sum<NT>(dsum, red);
     if (t == 0) p.dotp[(long)b * (p.dot_ld ? p.dot_ld : per) + tile + (long)p.ntile * zch] = tot;
   }
   if (COMB || UPD) {
-    const double tot = block_sum<512>(dsum2, red);
+    const double tot = block_sum<NT>(dsum2, red);
     if (t == 0) p.dotp2[(long)b * (p.dot_ld ? p.dot_ld : per) + tile + (long)p.ntile * zch] = tot;
   }
   if (NORMS || UPD) {
-    const double tot = block_sum<512>(dsum3, red);
+    const double tot = block_sum<NT>(dsum3, red);
     if (t == 0) p.dotp3[(long)b * (p.dot_ld ? p.dot_ld : per) + tile + (long)p.ntile * zch] = tot;
   }
   if (MAXES) {
-    const double m = block_max<512>(cmx, red);
+    const double m = block_max<NT>(cmx, red);
     if (t == 0) atomicMax(p.cmax + b, (unsigned long long)__double_as_longlong(m));
   }
   if (!NORMS && p.omax) {  // non-negative doubles order like their bit patterns
-    const double m = block_max<512>(amax, red);
+    const double m = block_max<NT>(amax, red);
     if (t == 0) atomicMax(p.omax + b, (unsigned long long)__double_as_longlong(m));
   }
 }
 
-// waves per SIMD the register budget is sized for: 4 where the z-columns fit in 128 VGPRs
-// (a 512-thread block is 2 waves per SIMD, so only even counts matter)
+// waves per SIMD the register budget of a 512-thread block is sized for: 4 where the z-columns fit
+// in 128 VGPRs (such a block is 2 waves per SIMD, so only even counts matter)
 template <int NF, int P, int MODE>
 constexpr int stencil_waves() {
   if (NF > 4) return 2;
@@ -424,10 +438,16 @@ constexpr int stencil_waves() {
   return P <= 2 ? 4 : 2;
 }
 
+// planes of loads in flight: two where a second set of registers fits (one point per thread)
 template <int NF, int P, int MODE>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(stencil_waves<NF, P, MODE>()))) void k_stencil_lds(SL p) {
+constexpr int stencil_depth() {
+  return P == 1 && NF <= 4 && MODE != 1 && MODE != 2 && MODE != 6 ? 2 : 1;
+}
+
+template <int NF, int P, int MODE, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(NT > 512 ? 4 : stencil_waves<NF, P, MODE>()))) void k_stencil_lds(SL p) {
   extern __shared__ double lds[];
-  __shared__ double red[8];
+  __shared__ double red[NT / 64];
   const int L = blockIdx.x, xcd = L & 7, j = L >> 3;
   const int per = p.ntile * p.nzch;
   int b, rem;
@@ -441,7 +461,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(stencil_wav
     b = (int)(it / per);
     rem = (int)(it % per);
   }
-  stencil_block<NF, P, MODE>(p, b, rem % p.ntile, rem / p.ntile, lds, red);
+  stencil_block<NF, P, MODE, stencil_depth<NF, P, MODE>(), NT>(p, b, rem % p.ntile, rem / p.ntile, lds, red);
 }
 
 // Several independent grids in one persistent launch: work-group g takes items g, g + G,
@@ -459,7 +479,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(NF <= 4 && 
     const long j = it - start[s];
     const int per = p.ntile * p.nzch;
     const int b = (int)(j / per), rem = (int)(j % per);
-    stencil_block<NF, P, MODE>(p, b, rem % p.ntile, rem / p.ntile, lds, red);
+    stencil_block<NF, P, MODE, 1, 512>(p, b, rem % p.ntile, rem / p.ntile, lds, red);
     __syncthreads();  // the next item reuses the LDS slab
   }
 }
@@ -1177,20 +1197,30 @@ void fd_coefficients(int nf, double *acfd) { fd_weights(nf, acfd); }
 
 // Tile plan of the LDS kernel for grid g and nb bands (nx <= 256).
 struct LdsPlan {
-  int TY, ntile, nzch, zc, P;
+  int TY, ntile, nzch, zc, P, nt;
 };
-static LdsPlan lds_plan(const Grid &g, int NF, int nb, int force_p = 0) {
+// A work-group is 1024 threads where the stencil reaches two to four rows and the bands fill the
+// chip: its tile has twice the rows of a 512-thread one, so the 2 NF halo rows, which come from L2
+// for every tile, cost half as much per point.  Measured at 128^3 x 1024 / 96^3 x 512 bands, per
+// launch: plain form 10.6 -> 10.0 / 2.29 -> 2.31 ms; combination form (512 threads: one point per
+// thread, one plane of loads in flight) 14.6 / 3.42 ms, with two planes in flight 13.9 / 3.16, with
+// 1024 threads 13.2 / 2.82, and with two points per thread (which 512 threads have no registers for)
+// 12.1 / 2.72.  A radius-1 form has too little halo to gain, a wider one no registers, and few
+// bands need the parallelism.
+static LdsPlan lds_plan(const Grid &g, int NF, int nb, int force_p = 0, bool comb = false, bool wide = true) {
   LdsPlan L;
   // P points per thread (param "stencil_p": 1, 2 or 4; default 2), TY rows of nx points
-  int pp = force_p > 0 ? force_p : (int)param("stencil_p", 2.0);
+  int pp = force_p > 0 ? force_p : comb ? (int)param("comb_p", 2.0) : (int)param("stencil_p", 2.0);
   pp = pp >= 4 ? 4 : (pp >= 2 ? 2 : 1);
   if (NF > 4) pp = 1;  // the z-column of a wide stencil leaves registers for one point
   // few bands (a Poisson solve): one point per thread and short z-ranges, for parallelism
   const bool few = (long)nb * ((g.ny * g.nx + 512 * pp - 1) / (512 * pp)) < 1024;
   if (few && force_p == 0) pp = 1;
-  L.TY = std::max(1, std::min(g.ny, 512 * pp / g.nx));
+  L.nt = wide && !few && pp <= 2 && NF >= 2 && NF <= 4 ? 1024 : 512;
+  if (comb && L.nt == 512) pp = 1;
+  L.TY = std::max(1, std::min(g.ny, L.nt * pp / g.nx));
   L.ntile = (g.ny + L.TY - 1) / L.TY;
-  L.P = (g.nx * L.TY + 511) / 512;
+  L.P = (g.nx * L.TY + L.nt - 1) / L.nt;
   if (L.P == 3) L.P = 4;
   // z-ranges: enough blocks to fill the chip, each range at least 4 NF planes (2 NF planes
   // for few bands: the extra warm-up planes are re-read from cache)
@@ -1204,12 +1234,8 @@ static LdsPlan lds_plan(const Grid &g, int NF, int nb, int force_p = 0) {
 }
 static bool lds_ok(const Grid &g) { return g.nx <= 256 && g.nx >= 8 && g.ny >= 8 && g.nz >= 8; }
 
-// points per thread of the combination-form stencil (param comb_p, default 1: measured faster
-// than 2 points at two waves per SIMD)
-static int comb_points() { return (int)param("comb_p", 1.0); }
-
 int stencil_parts_lds(const Grid &g, int NF, int nb, bool comb = false) {
-  LdsPlan L = lds_plan(g, NF, nb, comb ? comb_points() : 0);
+  LdsPlan L = lds_plan(g, NF, nb, 0, comb);
   return L.ntile * L.nzch;
 }
 
@@ -1228,18 +1254,23 @@ static void launch_lds_nf(const SL &p, const LdsPlan &L, int nb, hipStream_t s) 
   const long per = (long)L.ntile * L.nzch;
   // nb >= 8: band groups of 8 (one band per XCD); fewer: the items split over the 8 XCDs
   const unsigned grid = (unsigned)(nb >= 8 ? (long)(nb + 7) / 8 * 8 * per : 8 * ((nb * per + 7) / 8));
+  if constexpr (NF >= 2 && NF <= 4 && MODE != 1 && MODE != 6) {
+    if (L.nt == 1024) {
+      if (L.P == 1) hipLaunchKernelGGL((k_stencil_lds<NF, 1, MODE, 1024>), dim3(grid), dim3(1024), shm, s, p);
+      else hipLaunchKernelGGL((k_stencil_lds<NF, 2, MODE, 1024>), dim3(grid), dim3(1024), shm, s, p);
+      return;
+    }
+  }
   switch (L.P) {
-    case 1: hipLaunchKernelGGL((k_stencil_lds<NF, 1, MODE>), dim3(grid), dim3(512), shm, s, p); break;
-    case 2: hipLaunchKernelGGL((k_stencil_lds<NF, 2, MODE>), dim3(grid), dim3(512), shm, s, p); break;
-    default: hipLaunchKernelGGL((k_stencil_lds<NF, 4, MODE>), dim3(grid), dim3(512), shm, s, p); break;
+    case 1: hipLaunchKernelGGL((k_stencil_lds<NF, 1, MODE, 512>), dim3(grid), dim3(512), shm, s, p); break;
+    case 2: hipLaunchKernelGGL((k_stencil_lds<NF, 2, MODE, 512>), dim3(grid), dim3(512), shm, s, p); break;
+    default: hipLaunchKernelGGL((k_stencil_lds<NF, 4, MODE, 512>), dim3(grid), dim3(512), shm, s, p); break;
   }
 }
 
 // Generic LDS launch: coefficients in p; in2/eps for the residual mode.
 static void launch_lds(SL &p, const Grid &g, int NF, int nb, bool res, hipStream_t s) {
-  // the combination form prefetches two more values per point (the second band and its H):
-  // one point per thread keeps it within the register budget of four waves per SIMD
-  LdsPlan L = lds_plan(g, NF, nb, p.ca ? comb_points() : 0);
+  LdsPlan L = lds_plan(g, NF, nb, 0, p.ca != nullptr);
   if (L.P > 4) throw Error(1, "stencil tile does not fit the thread block");
   p.TY = L.TY; p.ntile = L.ntile; p.nzch = L.nzch; p.zc = L.zc; p.nbands = nb;
   if (res) {
@@ -1435,7 +1466,7 @@ StencilBatchPlan plan_stencil_batch(const std::vector<StencilCall> &calls, bool 
       q.c0 = q.cx[0] + q.cy[0] + q.cz[0];
     }
     // whole z-columns unless the system has too few tiles to share the chip
-    LdsPlan L = lds_plan(g, nf, c.nb, b.P);
+    LdsPlan L = lds_plan(g, nf, c.nb, b.P, false, false);
     L.zc = g.nz;
     L.nzch = 1;
     while ((long)c.nb * L.ntile * L.nzch < 64 && g.nz / (L.nzch * 2) >= 2 * nf) {
@@ -1462,7 +1493,7 @@ StencilBatchPlan plan_stencil_batch(const std::vector<StencilCall> &calls, bool 
 
 // parts per band of system i's stencil partial sums in a batch plan (tiles x z-ranges)
 long stencil_batch_parts(const Grid &g, int nf, int nb, int P) {
-  LdsPlan L = lds_plan(g, nf, nb, P);
+  LdsPlan L = lds_plan(g, nf, nb, P, false, false);
   int nzch = 1, zc = g.nz;
   while ((long)nb * L.ntile * nzch < 64 && g.nz / (nzch * 2) >= 2 * nf) {
     nzch *= 2;

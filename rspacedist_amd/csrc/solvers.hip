@@ -414,7 +414,7 @@ __global__ __launch_bounds__(64) void k_force_sum(const int *act, const int *is_
 
 // rho(:,s) (=|+=) scale sum_l f_l psi_l^2 over all bands, band order (scf_charge8f.F90:303-318):
 // one launch, eight bands' loads in flight per point (with one launch per 64 bands rho was
-// cleared, read and written between them; 40^3 x 32: 25.8 -> 23 us for the call)
+// cleared, read and written between them; 40^3 x 32: 26 -> 18 us for the call)
 __global__ __launch_bounds__(256) void k_charge(long n, int nb, const double *psi, long ld, const double *f,
                                                 double scale, int add, double *rho) {
   const long i = blockIdx.x * (long)blockDim.x + threadIdx.x;
@@ -955,10 +955,10 @@ static void dgemm(rocblas_operation ta, rocblas_operation tb, int m, int n, int 
 
 // C(M x M) = alpha A^T B + beta C in FP64 where the consumer reads one triangle only (tri 1:
 // on and below the diagonal, 2: on and above).  Where the matrix-core kernel does not apply, the
-// b (b + 1) / 2 blocks of a b x b partition
-// that hold it, b = param "gram_blocks" (default 4) limited to blocks of at least 256 columns
-// (narrower blocks ran slower than the full product).  At 2,097,152 x 1024 x 1024: 44 ms
-// against 69 ms for the full dgemm.  Entries outside the blocks are left as they are.
+// b (b + 1) / 2 blocks of a b x b partition that hold it, b = param "gram_blocks" (default 4)
+// limited to blocks of at least 256 columns (narrower blocks ran slower than the full product).
+// At 2,097,152 x 1024 x 1024: 44 ms against 69 ms for the full dgemm.  Entries outside the blocks
+// are left as they are.
 static void dgemm_tn_tri(int M, long K, double alpha, const double *A, long lda, const double *B,
                          long ldb, double beta, double *C, long ldc, int tri) {
   if (gemm_f64_tn(M, M, K, alpha, A, lda, B, ldb, beta, C, ldc, tri, lib().stream)) return;
