@@ -1199,15 +1199,15 @@ void fd_coefficients(int nf, double *acfd) { fd_weights(nf, acfd); }
 struct LdsPlan {
   int TY, ntile, nzch, zc, P, nt;
 };
-// A work-group is 1024 threads where the stencil reaches two to four rows and the bands fill the
-// chip: its tile has twice the rows of a 512-thread one, so the 2 NF halo rows, which come from L2
-// for every tile, cost half as much per point.  Measured at 128^3 x 1024 / 96^3 x 512 bands, per
-// launch: plain form 10.6 -> 10.0 / 2.29 -> 2.31 ms; combination form (512 threads: one point per
-// thread, one plane of loads in flight) 14.6 / 3.42 ms, with two planes in flight 13.9 / 3.16, with
-// 1024 threads 13.2 / 2.82, and with two points per thread (which 512 threads have no registers for)
-// 12.1 / 2.72.  A radius-1 form has too little halo to gain, a wider one no registers, and few
-// bands need the parallelism.
-static LdsPlan lds_plan(const Grid &g, int NF, int nb, int force_p = 0, bool comb = false, bool wide = true) {
+// The combination form's work-group is 1024 threads where the stencil reaches two to four rows and
+// the bands fill the chip: its tile has more rows, so the 2 NF halo rows, which come from L2 for
+// every tile, cost less per point, and a thread holds half as many of their values.  Per launch at
+// 128^3 x 1024 / 96^3 x 512 bands: 512 threads with one point per thread and one plane of loads in
+// flight 14.6 / 3.42 ms, with two planes in flight 13.9 / 3.16, 1024 threads 13.2 / 2.82, and with
+// two points per thread (which 512 threads have no registers for) 12.1 / 2.72.  The plain form has
+// two points per thread with 512 already and gains little (10.6 -> 10.0 / 2.29 -> 2.31) or, without
+// its store, loses; a wider stencil has no registers, and few bands need the parallelism.
+static LdsPlan lds_plan(const Grid &g, int NF, int nb, int force_p = 0, bool comb = false) {
   LdsPlan L;
   // P points per thread (param "stencil_p": 1, 2 or 4; default 2), TY rows of nx points
   int pp = force_p > 0 ? force_p : comb ? (int)param("comb_p", 2.0) : (int)param("stencil_p", 2.0);
@@ -1216,7 +1216,7 @@ static LdsPlan lds_plan(const Grid &g, int NF, int nb, int force_p = 0, bool com
   // few bands (a Poisson solve): one point per thread and short z-ranges, for parallelism
   const bool few = (long)nb * ((g.ny * g.nx + 512 * pp - 1) / (512 * pp)) < 1024;
   if (few && force_p == 0) pp = 1;
-  L.nt = wide && !few && pp <= 2 && NF >= 2 && NF <= 4 ? 1024 : 512;
+  L.nt = comb && !few && pp <= 2 && NF >= 2 && NF <= 4 ? 1024 : 512;
   if (comb && L.nt == 512) pp = 1;
   L.TY = std::max(1, std::min(g.ny, L.nt * pp / g.nx));
   L.ntile = (g.ny + L.TY - 1) / L.TY;
@@ -1254,7 +1254,7 @@ static void launch_lds_nf(const SL &p, const LdsPlan &L, int nb, hipStream_t s) 
   const long per = (long)L.ntile * L.nzch;
   // nb >= 8: band groups of 8 (one band per XCD); fewer: the items split over the 8 XCDs
   const unsigned grid = (unsigned)(nb >= 8 ? (long)(nb + 7) / 8 * 8 * per : 8 * ((nb * per + 7) / 8));
-  if constexpr (NF >= 2 && NF <= 4 && MODE != 1 && MODE != 6) {
+  if constexpr (NF >= 2 && NF <= 4 && (MODE == 2 || MODE == 5)) {
     if (L.nt == 1024) {
       if (L.P == 1) hipLaunchKernelGGL((k_stencil_lds<NF, 1, MODE, 1024>), dim3(grid), dim3(1024), shm, s, p);
       else hipLaunchKernelGGL((k_stencil_lds<NF, 2, MODE, 1024>), dim3(grid), dim3(1024), shm, s, p);
@@ -1466,7 +1466,7 @@ StencilBatchPlan plan_stencil_batch(const std::vector<StencilCall> &calls, bool 
       q.c0 = q.cx[0] + q.cy[0] + q.cz[0];
     }
     // whole z-columns unless the system has too few tiles to share the chip
-    LdsPlan L = lds_plan(g, nf, c.nb, b.P, false, false);
+    LdsPlan L = lds_plan(g, nf, c.nb, b.P);
     L.zc = g.nz;
     L.nzch = 1;
     while ((long)c.nb * L.ntile * L.nzch < 64 && g.nz / (L.nzch * 2) >= 2 * nf) {
@@ -1493,7 +1493,7 @@ StencilBatchPlan plan_stencil_batch(const std::vector<StencilCall> &calls, bool 
 
 // parts per band of system i's stencil partial sums in a batch plan (tiles x z-ranges)
 long stencil_batch_parts(const Grid &g, int nf, int nb, int P) {
-  LdsPlan L = lds_plan(g, nf, nb, P, false, false);
+  LdsPlan L = lds_plan(g, nf, nb, P);
   int nzch = 1, zc = g.nz;
   while ((long)nb * L.ntile * nzch < 64 && g.nz / (nzch * 2) >= 2 * nf) {
     nzch *= 2;
