@@ -650,6 +650,7 @@ __global__ __launch_bounds__(256) void k_gather_mfma(GatherArgs g) {
   __shared__ double red[4][16 * RT * 16];
   const int a = blockIdx.y, t = threadIdx.x, lane = t & 63, w = t >> 6, q = lane >> 4, c16 = lane & 15;
   const int slot = g.act[5 * a], natinf = g.act[5 * a + 1], iprj = g.act[5 * a + 2];
+  if (iprj == 0) return;  // uniform: a species without projectors has no row, and nothing to write
   const int b0 = blockIdx.x * 16, nrow = g.ntab * iprj;
   const double *v = g.psi + g.ld * min(b0 + c16, g.nb - 1);  // bands past the end: results unused
   const int *ls = g.lst + (long)g.num_list * slot;

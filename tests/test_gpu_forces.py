@@ -79,3 +79,63 @@ def test_gather_edges(kk, nprj, bands, n):
         w = psi[s.lstvec2[:m, a] - 1]
         err = np.abs(rp[:, a] - tabs[0][:m, :, a].T @ w)
         assert np.all(err <= kappa * (s.num_list + s.npts) * 2.0 ** -53 * (np.abs(tabs[0][:m, :, a]).T @ np.abs(w)))
+
+
+@pytest.mark.parametrize("bands", [7, 8, 40])
+def test_species_with_different_projector_counts(kk, orc, bands):
+    """Atoms of three species with 0, 9 and 4 projectors on one table: the atom without projectors
+    contributes nothing and leaves its neighbours' <p|psi> alone, through the orthonormalisation,
+    the adjoint's four-table pass, the band energy, the forces and both band solvers.  Bounds of
+    the sums as in test_gather_edges and above; the two band solvers against the oracle after one
+    iteration, to the rounding of test_gpu_seqcg's iterates (1e-8 of the largest entry)."""
+    nprj, natom = np.array([0, 9, 4], dtype=np.int32), 5
+    s = synth.make_system(12, 0.4, natom, bands, seed=bands)
+    assert s.natinf.min() > 16
+    rng = np.random.default_rng(bands)
+    spe = np.array([1, 2, 3, 1, 2], dtype=np.int32)
+    count = nprj[spe - 1]
+    tabs = [rng.standard_normal((s.num_list, 9, natom)) for _ in range(4)]
+    dij = rng.standard_normal((9, 9, 1, natom))
+    dij = dij + dij.transpose(1, 0, 2, 3)
+    for a, c in enumerate(count):  # zeros past a species' count
+        dij[c:, :, :, a] = dij[:, c:, :, a] = 0.0
+        for t in tabs:
+            t[:, c:, a] = 0.0
+    tabs, dij = [np.asfortranarray(0.01 * t) for t in tabs], np.asfortranarray(0.1 * dij)
+    kw = synth.abi_args(s, num_spe=3, nprj=nprj, indspe=spe, ntyppp=np.full(3, synth.KEY_PP_PAW, dtype=np.int32),
+                        sss=np.zeros((9, 9, 3), order="F"), vnlocp=tabs[0], dij=dij)
+    f, e = rng.random(bands), rng.standard_normal(bands)
+    psi0 = synth.smooth_bands(synth.random_bands(s), s.n, s.h, width=0.6 * s.h)
+    out = []
+    for call in (kk.call, orc.call):
+        psi, rp = psi0.copy(order="F"), np.zeros((9, natom, bands), order="F")
+        call("orthogonalization_r", **kw, nflag=1, svecre=psi, ssvre=psi.copy(order="F"), rspsep=rp)
+        fa = [np.zeros(natom) for _ in range(3)]
+        call("force_eig_r", **kw, svecre=psi, sval=e, fnele=f, fatx=fa[0], faty=fa[1], fatz=fa[2])
+        st = dict(svecre=psi.copy(order="F"), ssvre=psi.copy(order="F"), hsvre=np.zeros_like(psi, order="F"),
+                  rspsep=rp.copy(order="F"), sval=np.zeros(bands), residual_states=np.zeros(bands))
+        call("kscg_r", **dict(kw, nsdmax=1, epssd=1e-14), **st)
+        out.append(dict(st, psi=psi, rp=rp, force=np.stack(fa)))
+    for k in ("psi", "force"):
+        np.testing.assert_allclose(out[0][k], out[1][k], rtol=0, atol=1e-11 * np.abs(out[1][k]).max(), err_msg=k)
+    for k in ("svecre", "hsvre", "rspsep", "sval"):
+        np.testing.assert_allclose(out[0][k], out[1][k], rtol=0, atol=1e-8 * np.abs(out[1][k]).max(), err_msg=k)
+    psi, rp = out[0]["psi"], out[0]["rp"]
+    eb, dedv, dedr = np.zeros(bands), np.zeros(s.npts), np.zeros((natom, 3), order="F")
+    kk.call("band_energy_r", **kw, svecre=psi, eband=eb)
+    kk.call("energy_adjoint_r", **kw, dvnlocp=np.asfortranarray(np.stack(tabs[1:], axis=-1)), svecre=psi, fnele=f,
+            dedv=dedv, dedr=dedr)
+    want, bound = np.zeros((natom, 3)), np.zeros((natom, 3))
+    for a, c in enumerate(count):
+        m = s.natinf[a]
+        w, D = psi[s.lstvec2[:m, a] - 1], dij[:c, :c, 0, a]
+        r = [t[:m, :c, a].T @ w for t in tabs]
+        ra = [np.abs(t[:m, :c, a]).T @ np.abs(w) for t in tabs]
+        assert np.all(np.abs(rp[:c, a] - r[0]) <= 50.0 * (s.num_list + s.npts) * 2.0 ** -53 * ra[0])
+        assert not rp[c:, a].any()
+        for d in range(3):
+            want[a, d] = 2 * np.einsum("l,il,ij,jl->", f, r[1 + d], D, r[0], optimize=True)
+            bound[a, d] = 2 * np.einsum("l,il,ij,jl->", f, ra[1 + d], np.abs(D), ra[0], optimize=True)
+    assert np.all(np.abs(dedr - want) <= (2 * s.num_list + 81 + bands) * 2.0 ** -53 * bound)
+    # one iteration's eigenvalue estimate is <psi|H|psi> of the orthonormal bands it starts from
+    np.testing.assert_allclose(eb[0], out[0]["sval"][0], rtol=0, atol=1e-11 * np.abs(eb).max())
