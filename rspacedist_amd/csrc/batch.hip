@@ -745,6 +745,7 @@ void prepare(Batch &B) {
   std::vector<int> st0(3L * ns, 0);
   HIPCK(hipMemcpy(B.hstate, st0.data(), sizeof(int) * st0.size(), hipMemcpyHostToDevice));
   autotune(B, s);
+  B.hcg.clear();  // a preparation that failed part-way is repeated by the next step
   std::vector<BandRef> br(nbt);
   std::vector<HSys> hs(ns);
   for (int i = 0; i < ns; i++) {

@@ -123,6 +123,34 @@ def test_orthonormalisation_tile_edges(kk):
         assert np.abs(s.dv * got.T @ got - np.eye(s.nbands)).max() < 1e-12
 
 
+def test_step_after_a_preparation_that_failed(kk):
+    """A first step refused for a system of more than 128 bands, then one without the
+    orthonormalisation that refuses it: the step of a batch that never failed, up to the rounding of
+    the sums (each preparation chooses its own stencil tile), ~1e-15 an iteration."""
+    shapes, out = [(9, 3), (8, 130), (12, 5)], []
+    for fail in (True, False):
+        systems = []
+        for n, m in shapes:
+            s = synth.make_system(n, 0.35, 2, m, seed=10 * n + m)
+            q, _ = np.linalg.qr(synth.random_bands(s))
+            systems.append((s, np.asfortranarray(q / np.sqrt(s.dv))))
+        b = _batch(systems)
+        if fail:
+            with pytest.raises(kk.KukanError, match="at most 128 bands"):
+                b.step(ncgmax=7)
+        kk.set_param("batch_ortho", 0)
+        try:
+            b.step(ncgmax=7, epsvh=1e-30)
+        finally:
+            kk.set_param("batch_ortho", 1)
+        out.append([b.get(i) for i in range(len(shapes))])
+        b.close()
+    for got, want in zip(*out):
+        assert got[3] == want[3] == 7
+        for x, y in zip(got[:3], want[:3]):
+            np.testing.assert_allclose(x, y, rtol=0, atol=1e-11 * np.abs(y).max())
+
+
 def test_batching_config_48_systems(kk):
     """The 48-system configuration (sizes in {32,48,64,80}^3, 16..128 bands, 2..24 atoms):
     batched (persistent stencil launches + graph replays) vs the per-system launch loop, same
