@@ -460,6 +460,7 @@ struct Batch {
   int *hstate = nullptr;     // 3 per system
   std::vector<HcgArgs> hcg;  // the Hartree iteration's arguments, their device copy and units
   HcgArgs *hcg_dev = nullptr;
+  bool hcg_sent = false;     // hcg_dev holds hcg
   int2 *hdir = nullptr, *hupd = nullptr;
   std::vector<int> hd0, hu0;  // each system's first unit (ns + 1)
   std::vector<void *> owned;
@@ -648,12 +649,14 @@ void hartree_solve(Batch &B, int s0, int s1, bool batched, int ncgmax, hipStream
 
 // The iteration's rule of this step into the device table
 void hartree_rule(Batch &B, int ncgmax, double eps) {
-  if (B.hcg[0].ncgmax == ncgmax && B.hcg[0].eps == eps) return;
+  if (B.hcg_sent && B.hcg[0].ncgmax == ncgmax && B.hcg[0].eps == eps) return;
+  B.hcg_sent = false;
   for (HcgArgs &a : B.hcg) {
     a.ncgmax = ncgmax;
     a.eps = eps;
   }
   HIPCK(hipMemcpy(B.hcg_dev, B.hcg.data(), sizeof(HcgArgs) * B.hcg.size(), hipMemcpyHostToDevice));
+  B.hcg_sent = true;
 }
 
 template <class F>
@@ -746,6 +749,7 @@ void prepare(Batch &B) {
   HIPCK(hipMemcpy(B.hstate, st0.data(), sizeof(int) * st0.size(), hipMemcpyHostToDevice));
   autotune(B, s);
   B.hcg.clear();  // a preparation that failed part-way is repeated by the next step
+  B.hcg_sent = false;
   std::vector<BandRef> br(nbt);
   std::vector<HSys> hs(ns);
   for (int i = 0; i < ns; i++) {
