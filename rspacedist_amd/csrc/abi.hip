@@ -692,8 +692,10 @@ int kukan_scf_charge_smt_r(int neigmx, int nums, int nspv, int numk, int ncpx, i
   Arr F(fnele, (size_t)nall * D, Arr::In);
   Arr Ps(svecre, (size_t)n * nall * D, Arr::In);
   Arr Rho(rhosmt, (size_t)n * nspv * D, Arr::Out);
-  // channels without a spin of their own stay zero; the others start with their first contribution
-  if (nspv > nums) launch_fill(n * (nspv - nums), 0.0, Rho.d() + (size_t)n * nums, lib().stream);
+  // channels without a spin of their own, or without a k-point, are zero; the others start with
+  // their first contribution
+  const int given = numk > 0 ? std::min(nums, nspv) : 0;
+  if (nspv > given) launch_fill(n * (nspv - given), 0.0, Rho.d() + (size_t)n * given, lib().stream);
   for (int ns = 1; ns <= nums; ns++) {
     const int nsr = std::min(ns, nspv);
     for (int nk = 1; nk <= numk; nk++) {

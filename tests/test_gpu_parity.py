@@ -537,3 +537,20 @@ def test_hpsi_tiled_path_ragged_grid(kk, orc, nperi):
     g, o = both(kk, orc, "rayleighritz_r", arr, **kw)
     np.testing.assert_allclose(g["sval"], o["sval"], rtol=1e-11, atol=1e-10)
     np.testing.assert_allclose(g["svecre"], o["svecre"], atol=1e-8 * np.abs(o["svecre"]).max())
+
+
+@pytest.mark.parametrize("nums,nspv,numk,m", [(1, 1, 1, 1), (1, 2, 1, 9), (2, 1, 2, 16), (2, 2, 3, 7), (2, 2, 0, 3),
+                                              (1, 1, 0, 3)])
+def test_charge_channels(kk, nums, nspv, numk, m):
+    """Every channel of the density is written, whatever it held: the sum of its spins and k-points
+    (both spins where there is one channel), zero without any.  A sum of numk m terms or twice as
+    many is off by at most that many 2^-53 of itself."""
+    rng = np.random.default_rng(nums + 10 * numk)
+    psi, f = rng.standard_normal((numk, nums, m, 6 * 5 * 7)), rng.random((numk, nums, m))
+    rho = kk.DeviceArray.from_numpy(np.full(nspv * 210, np.nan))
+    kk.call("scf_charge_smt_r", neigmx=m, nums=nums, nspv=nspv, numk=numk, ncpx=6, ncpy=5, ncpz=7,
+            fnele=np.append(f, 0.0), svecre=np.append(psi, 0.0), rhosmt=rho)
+    want = np.zeros((nspv, 210))
+    for s in range(nums):
+        want[min(s, nspv - 1)] += (f[:, s, :, None] * psi[:, s] ** 2).sum(axis=(0, 1))
+    np.testing.assert_allclose(rho.numpy().reshape(nspv, 210), want, rtol=(2 * numk * m + 4) * 2.0 ** -53, atol=0)
