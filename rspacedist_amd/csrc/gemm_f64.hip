@@ -140,6 +140,16 @@ __global__ __launch_bounds__(256) void k_tn_f64(TNArgs a) {
 // columns.
 typedef double d2 __attribute__((ext_vector_type(2)));
 #define GF_LDS(x) ((__attribute__((address_space(3))) void *)(x))
+// Between two steps of a ring of two slots: this wave's loads into the next slot have landed and its
+// reads of the other slot have returned (vmcnt 0 and lgkmcnt 0), then every wave's.  The reads have
+// to be waited for here: the barrier alone would let another wave's loads overwrite a slot whose
+// values the compiler need not have used yet.
+__device__ inline void ring_step() {
+  __builtin_amdgcn_s_waitcnt(0x0070);
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
 __global__ __launch_bounds__(256, 2) void k_tn_f64_lds(TNArgs a) {
   constexpr int WT = 4, TM = 128;
   __shared__ __attribute__((aligned(1024))) char ring[2][2][TM * 128];  // [slot][A, B]
@@ -190,10 +200,7 @@ __global__ __launch_bounds__(256, 2) void k_tn_f64_lds(TNArgs a) {
   const int la = 128 * (64 * (w & 1) + c16) + 16 * (q ^ (c16 >> 1)), lb = 128 * (64 * (w >> 1) + c16) + 16 * (q ^ (c16 >> 1));
   if (nf > 0) issue(0);
   for (int st = 0; st < nf; st++) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's part of the step has landed
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();        // and every wave's; the other slot has been read
-    asm volatile("" ::: "memory");
+    ring_step();
     if (st + 1 < nf) issue(st + 1);
     const char *A = ring[st & 1][0], *B = ring[st & 1][1];
     d2 x[2][WT], y[2][WT];
@@ -369,10 +376,7 @@ __global__ __launch_bounds__(256, 2) void k_nn_f64(NNArgs64 a) {
   const int lc = 128 * (64 * wi + c16) + 16 * (q ^ (c16 >> 1)), lx = 2048 * q + 512 * wj + 16 * c16;
   issue(0);
   for (int st = 0; st < nst; st++) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's part of the step has landed
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();        // and every wave's; the other slot has been read
-    asm volatile("" ::: "memory");
+    ring_step();
     if (st + 1 < nst) issue(st + 1);
     const char *X = ring[st & 1][0], *C = ring[st & 1][1];
     d2 x[2][2][2], y[2][4];
