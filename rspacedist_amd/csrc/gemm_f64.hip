@@ -400,21 +400,15 @@ __global__ __launch_bounds__(256, 2) void k_nn_f64(NNArgs64 a) {
             acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(y[h][i][s], x[h][s][j >> 1][j & 1], acc[i][j], 0, 0, 0);
   }
   // a wave's 16 columns x 64 points at a time; with beta the Y values of the next 16 columns are
-  // loaded while these are written
-  auto yptr = [&](int i, int r, int g) {
-    const int j = min(c0 + 64 * wi + 16 * i + q + 4 * r, a.M2 - 1);
-    return a.Y + a.ldy * j + min(r0 + 64 * wj + 32 * g + 2 * c16, (a.R - 1) & ~1L);
-  };
-  const bool odd = r0 + TM > a.R;  // the last row block may end inside a lane's pair of points
+  // loaded while these are written (past the last point or column: the last ones again, unused)
   d2 yo[2][4][2];
   auto fetch = [&](int i) {
 #pragma unroll
     for (int r = 0; r < 4; r++)
 #pragma unroll
       for (int g = 0; g < 2; g++) {
-        const double *y = yptr(i, r, g);
-        if (odd) yo[i & 1][r][g] = d2{y[0], y - a.Y + 1 < a.ldy * a.M2 - (a.ldy - a.R) ? y[1] : 0.0};
-        else yo[i & 1][r][g] = *(const d2 *)y;
+        const int j = min(c0 + 64 * wi + 16 * i + q + 4 * r, a.M2 - 1);
+        yo[i & 1][r][g] = *(const d2 *)(a.Y + a.ldy * j + min(r0 + 64 * wj + 32 * g + 2 * c16, a.R - 2));
       }
   };
   if (a.beta != 0.0) fetch(0);
@@ -430,9 +424,7 @@ __global__ __launch_bounds__(256, 2) void k_nn_f64(NNArgs64 a) {
         const long p = r0 + 64 * wj + 32 * g + 2 * c16;
         d2 v = {acc[i][2 * g][r], acc[i][2 * g + 1][r]};
         if (a.beta != 0.0) v += a.beta * yo[i & 1][r][g];
-        double *y = a.Y + a.ldy * j + p;
-        if (p + 1 < a.R) *(d2 *)y = v;
-        else if (p < a.R) *y = v[0];
+        if (p < a.R) *(d2 *)(a.Y + a.ldy * j + p) = v;
       }
     }
   }
@@ -442,9 +434,11 @@ __global__ __launch_bounds__(256, 2) void k_nn_f64(NNArgs64 a) {
 
 static bool aligned16(const void *p, long ld) { return (uintptr_t)p % 16 == 0 && ld % 2 == 0; }
 
+// R even: a lane loads and stores points in pairs (the bands' own length, so an odd one has columns
+// that are not 16-byte aligned either)
 static bool nn_ok(const double *X, long ldx, const double *Y, long ldy, long R, int K, int M2) {
-  return param("gemm_f64", 1.0) >= 1.0 && R > 0 && K > 0 && M2 > 0 && aligned16(X, ldx) && aligned16(Y, ldy) &&
-         ldx < (1L << 24) && K <= 16384;
+  return param("gemm_f64", 1.0) >= 1.0 && R > 0 && R % 2 == 0 && K > 0 && M2 > 0 && aligned16(X, ldx) &&
+         aligned16(Y, ldy) && ldx < (1L << 24) && K <= 16384;
 }
 
 static NNArgs64 nn_prepare(long R, int K, int M2, double alpha, const double *X, long ldx, const double *C,
