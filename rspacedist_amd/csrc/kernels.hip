@@ -1208,17 +1208,24 @@ struct LdsPlan {
 // two points per thread (which 512 threads have no registers for) 12.1 / 2.72.  The plain form has
 // two points per thread with 512 already and gains little (10.6 -> 10.0 / 2.29 -> 2.31) or, without
 // its store, loses; a wider stencil has no registers, and few bands need the parallelism.
-static LdsPlan lds_plan(const Grid &g, int NF, int nb, int force_p = 0, bool comb = false) {
+// Those are the symmetric form's times.  The general one (unsymmetric dij) also holds the second
+// band; with a stencil of four rows two points of it do not fit 128 VGPRs (10 are spilled) and it
+// keeps one.  Per launch at 128^3 x 1024 / 96^3 x 512 bands, 512 threads and one point / 1024 and
+// one / 1024 and two: four rows 16.5 / 16.1 / 19.9 and 3.72 / 3.52 / 4.75 ms, three 15.3 / 15.4 /
+// 14.8 and 3.47 / 3.40 / 3.28, two 14.2 / 14.9 / 13.4 and 3.25 / 3.32 / 3.00.
+static LdsPlan lds_plan(const Grid &g, int NF, int nb, int force_p = 0, Comb comb = Comb::none) {
   LdsPlan L;
   // P points per thread (param "stencil_p": 1, 2 or 4; default 2), TY rows of nx points
-  int pp = force_p > 0 ? force_p : comb ? (int)param("comb_p", 2.0) : (int)param("stencil_p", 2.0);
+  const bool cf = comb != Comb::none;
+  int pp = force_p > 0 ? force_p : cf ? (int)param("comb_p", 2.0) : (int)param("stencil_p", 2.0);
   pp = pp >= 4 ? 4 : (pp >= 2 ? 2 : 1);
   if (NF > 4) pp = 1;  // the z-column of a wide stencil leaves registers for one point
+  if (NF == 4 && comb == Comb::general) pp = 1;
   // few bands (a Poisson solve): one point per thread and short z-ranges, for parallelism
   const bool few = (long)nb * ((g.ny * g.nx + 512 * pp - 1) / (512 * pp)) < 1024;
   if (few && force_p == 0) pp = 1;
-  L.nt = comb && !few && pp <= 2 && NF >= 2 && NF <= 4 ? 1024 : 512;
-  if (comb && L.nt == 512) pp = 1;
+  L.nt = cf && !few && pp <= 2 && NF >= 2 && NF <= 4 ? 1024 : 512;
+  if (cf && L.nt == 512) pp = 1;
   L.TY = std::max(1, std::min(g.ny, L.nt * pp / g.nx));
   L.ntile = (g.ny + L.TY - 1) / L.TY;
   L.P = (g.nx * L.TY + L.nt - 1) / L.nt;
@@ -1235,7 +1242,7 @@ static LdsPlan lds_plan(const Grid &g, int NF, int nb, int force_p = 0, bool com
 }
 static bool lds_ok(const Grid &g) { return g.nx <= 256 && g.nx >= 8 && g.ny >= 8 && g.nz >= 8; }
 
-int stencil_parts_lds(const Grid &g, int NF, int nb, bool comb = false) {
+int stencil_parts_lds(const Grid &g, int NF, int nb, Comb comb = Comb::none) {
   LdsPlan L = lds_plan(g, NF, nb, 0, comb);
   return L.ntile * L.nzch;
 }
@@ -1257,9 +1264,14 @@ static void launch_lds_nf(const SL &p, const LdsPlan &L, int nb, hipStream_t s) 
   const unsigned grid = (unsigned)(nb >= 8 ? (long)(nb + 7) / 8 * 8 * per : 8 * ((nb * per + 7) / 8));
   if constexpr (NF >= 2 && NF <= 4 && (MODE == 2 || MODE == 5)) {
     if (L.nt == 1024) {
-      if (L.P == 1) hipLaunchKernelGGL((k_stencil_lds<NF, 1, MODE, 1024>), dim3(grid), dim3(1024), shm, s, p);
-      else hipLaunchKernelGGL((k_stencil_lds<NF, 2, MODE, 1024>), dim3(grid), dim3(1024), shm, s, p);
-      return;
+      if (L.P == 1) {
+        hipLaunchKernelGGL((k_stencil_lds<NF, 1, MODE, 1024>), dim3(grid), dim3(1024), shm, s, p);
+        return;
+      }
+      if constexpr (NF < 4 || MODE == 5) {
+        hipLaunchKernelGGL((k_stencil_lds<NF, 2, MODE, 1024>), dim3(grid), dim3(1024), shm, s, p);
+        return;
+      }
     }
   }
   switch (L.P) {
@@ -1271,7 +1283,7 @@ static void launch_lds_nf(const SL &p, const LdsPlan &L, int nb, hipStream_t s) 
 
 // Generic LDS launch: coefficients in p; in2/eps for the residual mode.
 static void launch_lds(SL &p, const Grid &g, int NF, int nb, bool res, hipStream_t s) {
-  LdsPlan L = lds_plan(g, NF, nb, 0, p.ca != nullptr);
+  LdsPlan L = lds_plan(g, NF, nb, 0, !p.ca ? Comb::none : p.in2 ? Comb::general : Comb::symmetric);
   if (L.P > 4) throw Error(1, "stencil tile does not fit the thread block");
   p.TY = L.TY; p.ntile = L.ntile; p.nzch = L.nzch; p.zc = L.zc; p.nbands = nb;
   if (res) {
@@ -1330,7 +1342,7 @@ bool stencil_band_fastest_coef(const Grid &g, bool halo_in) {
   return !halo_in && lds_ok(g) && param("stencil_lds", 1.0) >= 1.0;
 }
 
-int stencil_nparts(const Grid &g, int nf, int nb, bool comb) {
+int stencil_nparts(const Grid &g, int nf, int nb, Comb comb) {
   if (lds_ok(g) && param("stencil_lds", 1.0) >= 1.0) return stencil_parts_lds(g, nf, nb, comb);
   const int zc = 8;
   return (int)(nblk(g.nx, 64) * nblk(g.ny, 4) * nblk(g.nz, zc));
@@ -1393,8 +1405,8 @@ void launch_stencil(const StencilCall &c, hipStream_t s) {
     }
     if (c.pl && c.coef && c.pl->nent > 0) {  // nonlocal part: separate owner-computes pass
       const bool comb = c.ca != nullptr, sym = comb && !c.in2;
-      const long pld = c.dot_ld ? c.dot_ld : stencil_parts_lds(g, nf, c.nb, comb);
-      const int off = stencil_parts_lds(g, nf, c.nb, comb);
+      const int off = stencil_parts_lds(g, nf, c.nb, !comb ? Comb::none : sym ? Comb::symmetric : Comb::general);
+      const long pld = c.dot_ld ? c.dot_ld : off;
       if (c.rp && c.dot_partial && (!comb || sym || c.rp2)) {
         launch_expand_rows(*c.pl, c.coef, c.nb, c.out, c.ld_out, nullptr, 0, nullptr, 0, 0, s,
                            nullptr, nullptr, nullptr, nullptr, c.expand_max);

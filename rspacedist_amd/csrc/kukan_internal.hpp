@@ -207,8 +207,11 @@ void launch_stencil_batch(const StencilBatchPlan &b, int grid, hipStream_t s);
 void launch_stencil(const StencilCall &c, hipStream_t s);
 // true when launch_stencil takes the tiled path, whose projector pass reads band-fastest coef
 bool stencil_band_fastest_coef(const Grid &g, bool halo_in);
+// the forms of the combination stencil (out = ca H in + cb hin): with the second band read, or for a
+// symmetric H without it
+enum class Comb { none, symmetric, general };
 // partial-sum layout of launch_stencil's dot_partial: nb * nparts
-int stencil_nparts(const Grid &g, int nf, int nb, bool comb = false);  // comb: combination form
+int stencil_nparts(const Grid &g, int nf, int nb, Comb comb = Comb::none);
 // fused r = sign*(h - eps s), out = K r, optional per-band partials of <r|K r>
 void launch_precond_resid_dot(const Grid &g, const double *h, const double *sp, long ld,
                               const double *eps, double sign, double *out, int nb,

@@ -915,7 +915,7 @@ void Ctx::hpsi_comb(int ns, const double *veffs, const double *x, const double *
   const bool pdots = rpy && param("nl_proj_dots", 1.0) >= 1.0;
   // H symmetric (dij symmetric): <y|H p> = <H y|ca x> + cb <y|H y>, so y is not read
   const bool sym = pdots && eh && param("comb_sym", 1.0) >= 1.0 && dij_symmetric();
-  const int np = stencil_nparts(g, g.nf, nb, true) + (pdots ? 1 : expand_nparts(pl));
+  const int np = stencil_nparts(g, g.nf, nb, sym ? Comb::symmetric : Comb::general) + (pdots ? 1 : expand_nparts(pl));
   double *part = buf("hpsi.part", (size_t)2 * np * nb);
   launch_fill((long)2 * np * nb, 0.0, part, s);
   StencilCall c;
