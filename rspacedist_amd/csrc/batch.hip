@@ -217,7 +217,6 @@ inline unsigned nb_(long n, int t) { return (unsigned)((n + t - 1) / t); }
 // to 126 bands: Gram 2.44 -> 0.53 ms, factor and inverse 1.18 -> 0.16 ms, apply 2.14 -> 0.47 ms
 // (vector FMAs from LDS tiles, and a column of the inverse per thread, before).
 constexpr int OMAX = 128;  // bands per system (the Cholesky runs in 128 KB of LDS)
-constexpr int ONT = OMAX / 16;
 typedef double d4 __attribute__((ext_vector_type(4)));
 typedef double d4u __attribute__((ext_vector_type(4), aligned(8)));
 struct OSys {

@@ -1262,22 +1262,27 @@ static void launch_lds_nf(const SL &p, const LdsPlan &L, int nb, hipStream_t s) 
   const long per = (long)L.ntile * L.nzch;
   // nb >= 8: band groups of 8 (one band per XCD); fewer: the items split over the 8 XCDs
   const unsigned grid = (unsigned)(nb >= 8 ? (long)(nb + 7) / 8 * 8 * per : 8 * ((nb * per + 7) / 8));
-  if constexpr (NF >= 2 && NF <= 4 && (MODE == 2 || MODE == 5)) {
-    if (L.nt == 1024) {
-      if (L.P == 1) {
-        hipLaunchKernelGGL((k_stencil_lds<NF, 1, MODE, 1024>), dim3(grid), dim3(1024), shm, s, p);
-        return;
-      }
-      if constexpr (NF < 4 || MODE == 5) {
-        hipLaunchKernelGGL((k_stencil_lds<NF, 2, MODE, 1024>), dim3(grid), dim3(1024), shm, s, p);
-        return;
+  auto run = [&](auto points, auto threads) {
+    constexpr int P = decltype(points)::value, NT = decltype(threads)::value;
+    hipLaunchKernelGGL((k_stencil_lds<NF, P, MODE, NT>), dim3(grid), dim3(NT), shm, s, p);
+  };
+  using std::integral_constant;
+  if constexpr (MODE == 2 || MODE == 5) {  // the combination forms: what lds_plan gives them
+    if constexpr (NF >= 2 && NF <= 4) {
+      if (L.nt == 1024) {
+        if constexpr (NF < 4 || MODE == 5) {
+          if (L.P == 2) return run(integral_constant<int, 2>(), integral_constant<int, 1024>());
+        }
+        return run(integral_constant<int, 1>(), integral_constant<int, 1024>());
       }
     }
-  }
-  switch (L.P) {
-    case 1: hipLaunchKernelGGL((k_stencil_lds<NF, 1, MODE, 512>), dim3(grid), dim3(512), shm, s, p); break;
-    case 2: hipLaunchKernelGGL((k_stencil_lds<NF, 2, MODE, 512>), dim3(grid), dim3(512), shm, s, p); break;
-    default: hipLaunchKernelGGL((k_stencil_lds<NF, 4, MODE, 512>), dim3(grid), dim3(512), shm, s, p); break;
+    return run(integral_constant<int, 1>(), integral_constant<int, 512>());
+  } else {
+    switch (L.P) {
+      case 1: return run(integral_constant<int, 1>(), integral_constant<int, 512>());
+      case 2: return run(integral_constant<int, 2>(), integral_constant<int, 512>());
+      default: return run(integral_constant<int, 4>(), integral_constant<int, 512>());
+    }
   }
 }
 

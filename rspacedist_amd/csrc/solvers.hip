@@ -650,13 +650,6 @@ struct HPArgs {
   HcgBar *bar;
 };
 __device__ inline int hcgp_wrap(int v, int n) { return v < 0 ? v + n : (v >= n ? v - n : v); }  // |overshoot| < n
-// p at (X, Y, z) with the grid's boundary rule: periodic directions wrap, isolated ones are 0
-__device__ inline double hcgp_p(const HPArgs &a, int X, int Y, int z) {
-  if (X < 0 || X >= a.nx) { if (!a.px) return 0.0; X = hcgp_wrap(X, a.nx); }
-  if (Y < 0 || Y >= a.ny) { if (!a.py) return 0.0; Y = hcgp_wrap(Y, a.ny); }
-  if (z < 0 || z >= a.nz) { if (!a.pz) return 0.0; z = hcgp_wrap(z, a.nz); }
-  return hcgp_ld(a.p + (long)X + (long)a.nx * ((long)Y + (long)a.ny * z));
-}
 // nx, ny, nz are multiples of 16 (the host checks): every thread owns 16 grid points.  The
 // stencil stages the x / y halo of 8 planes at a time in LDS (one load latency per 8 planes)
 // and the z-halo of every column with the first 8.
