@@ -470,7 +470,14 @@ bool gemm_f64_nn_upper(long R, int K, int M2, double alpha, const double *X, lon
   return true;
 }
 
-bool apply_upper_ok(long R, int M, const double *X, long ldx) { return nn_ok(X, ldx, X, ldx, R, M, M); }
+// Against dtrsm, which needs no inverse of the factor (a whole orthonormalisation with either, own /
+// dtrsm): up to 32 bands dtrsm is one pass and the inverse costs more than the rest (262144 points x
+// 20: 323 / 244 us, x 48: 429 / 474; 884736 x 32: 505 / 469) except on the longest bands, where the
+// passes count (2097152 x 32: 970 / 1036, x 24: 880 / 793); on short bands the inverse is never
+// repaid (4096 x 500: 1901 / 1736, 13824 x 800: 3299 / 3099, 32768 x 200: 892 / 935).
+bool apply_upper_ok(long R, int M, const double *X, long ldx) {
+  return R >= 32768 && M > (R < (1L << 21) ? 32 : 24) && nn_ok(X, ldx, X, ldx, R, M, M);
+}
 
 void gemm_f64_apply_upper(long R, int M, double *X, long ldx, const double *C, long ldc, hipStream_t s) {
   NNArgs64 a = nn_prepare(R, M, M, 1.0, X, ldx, C, ldc, X, ldx, s);

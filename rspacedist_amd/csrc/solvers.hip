@@ -1129,8 +1129,8 @@ void cholqr(Ctx &c, int M, double *psi, double *spsi, double *rsp, double *hpsi,
   HIPCK(hipMemcpyAsync(&hinfo, info, sizeof(int), hipMemcpyDeviceToHost, c.s));
   sync();
   if (hinfo != 0) throw Error(2, "orthogonalization_r_01 (1): wf has negative norm");
-  // X <- X R^-1: as a triangular matrix-core product with R^-1 where that applies (2097152 x
-  // 1024: 39 ms against 43 for dtrsm, which multiplies in blocks too), else by dtrsm
+  // X <- X R^-1: as a triangular matrix-core product with R^-1 where that is the faster one (2097152
+  // x 1024: 39 ms against 43 for dtrsm, which multiplies in blocks too), else by dtrsm
   double *Ri = nullptr;
   auto inverse = [&]() {  // R^-1 in FP64 (upper triangular)
     if (Ri) return;

@@ -53,6 +53,24 @@ def test_orthogonalisation_triangles(kk, n, m):
     np.testing.assert_allclose(psi * np.sqrt(s.dv), q, rtol=0, atol=s.npts * 2.0 ** -53 * kappa)
 
 
+@pytest.mark.parametrize("dims,m", [((32, 32, 32), 32), ((32, 32, 32), 33), ((31, 32, 33), 40), ((32, 33, 34), 129),
+                                    ((46, 27, 31), 260)])
+def test_orthogonalisation_long_bands(kk, dims, m):
+    """As above for bands long and many enough (32768 points, more than 32) that the inverse factor
+    is applied by the matrix-core product instead of dtrsm: both sides of the line, one to three
+    column tiles, points that end inside a tile."""
+    s = synth.make_system(12, 0.4, 2, m, seed=m)
+    n = int(np.prod(dims))
+    psi0 = np.asfortranarray(np.random.default_rng(m).standard_normal((n, m)))
+    psi = psi0.copy(order="F")
+    kk.call("orthogonalization_r", **synth.abi_args(s, ncpx=dims[0], ncpy=dims[1], ncpz=dims[2]), nflag=1, svecre=psi,
+            ssvre=psi, rspsep=np.zeros((9, s.natom, m), order="F"))
+    bound = n * 2.0 ** -53 * np.linalg.cond(psi0) ** 2
+    np.testing.assert_allclose(psi.T @ psi * s.dv, np.eye(m), rtol=0, atol=bound)
+    q, r = np.linalg.qr(psi0 * np.sqrt(s.dv))
+    np.testing.assert_allclose(psi * np.sqrt(s.dv), q * np.sign(np.diag(r)), rtol=0, atol=bound)
+
+
 @pytest.mark.parametrize("m", [66, 130, 257])
 def test_block_cg_projection_triangle(kk, m):
     """One block-CG step in FP64 with the triangular projection product and with every product
