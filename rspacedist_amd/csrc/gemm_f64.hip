@@ -284,9 +284,9 @@ void tn_launch(TNArgs a, bool lds, double alpha, double beta, double *C, long ld
   a.nt1 = nt1;
   a.npair = a.tri ? nt1 * (nt1 + 1) / 2 : nt1 * nt2;
   // K-ranges: a multiple of 8 (one XCD each in turn), at least 256 deep, the count whose
-  // rounds of resident work-groups (WT 4: 1 per CU, 2: 4 per CU) times depth is least; 128
+  // rounds of resident work-groups (WT 4: 1 per CU, 2: 4, 1: 8) times depth is least; 128
   // stands for a range's own start and end
-  const long res = lds ? 64 : WT == 4 ? 32 : 128;  // per XCD
+  const long res = lds ? 64 : WT == 4 ? 32 : WT == 2 ? 128 : 256;  // per XCD
   long best = 0;
   double cost = 1e300;
   for (long nc = 8; nc <= 2048 && (nc == 8 || nc * 256 <= a.K + 2047); nc += 8) {
@@ -487,33 +487,49 @@ void gemm_f64_apply_upper(long R, int M, double *X, long ldx, const double *C, l
   HIPCK(hipGetLastError());
 }
 
-// Which TN kernel, from times at K = 262144 .. 2097152 (rocBLAS dgemm beside them):
-//  - at most 64 columns on one side: 64 x 64 tiles.  rocBLAS runs the whole K in one tile's
-//    work-group there: 64000 x 32 takes 10.3 ms against 0.034 ms, 884736 x 64 1.70 against 0.27;
+// Which TN kernel, from times at K = 512 .. 8000000 (rocBLAS dgemm beside them; its times jump between
+// neighbouring sizes, and many are ten times these):
+//  - at most 32 columns on both sides: 32 x 32 tiles;
+//  - at most 64 on one side: 64 x 64 tiles.  rocBLAS runs the whole K in one tile's work-group
+//    there: 64000 x 32 takes 10.3 ms against 0.034 ms, 884736 x 64 1.70 against 0.27;
 //  - 16-byte aligned columns: 128 x 128 tiles through LDS, 73-75 TFLOP/s from 384 columns on
 //    (884736 x 512: 6.34 ms against 8.0; its triangle 4.23 against 5.9 in 256-column blocks;
-//    2097152 x 1024, the triangle: 33.7 against 44.5);
+//    2097152 x 1024, the triangle: 33.7 against 44.5).  Past 128 columns a short K does not repay
+//    the eight K-ranges' partial tiles and the launch that adds them: 512 x 512 34 us against 25,
+//    768 x 768 52 against 41, but 1024 x 1000 67 against 73; with more than 144 tiles K has to be six
+//    times the columns (8192 x 2000 1075 against 915, 12000 x 2000 1538 against 1977), and a full
+//    square past 3072 is rocBLAS's (16384 x 4096 8.42 ms against 8.05);
 //  - otherwise (an odd column length): the direct 128 x 128 kernel where it is at least as fast
 //    as rocBLAS, up to 128 columns (253440 x 100: 0.18 against 40.6 ms), for a triangle up to 384
 //    (3.1 against 6.0 ms).
-static int tn_kind(int M1, int M2, long K, const double *A, long lda, const double *B, long ldb, int tri) {
-  if (param("gemm_f64", 1.0) < 1.0 || M1 <= 0 || M2 <= 0 || K <= 0 || std::max(lda, ldb) >= (1L << 24)) return 0;
-  const bool near = std::max(lda, ldb) < (1L << 22);  // the direct kernels' offsets within a tile
-  if (std::min(M1, M2) <= 64 && near) return 1;
-  if (aligned16(A, lda) && aligned16(B, ldb)) return 2;
-  return near && std::max(M1, M2) <= (tri && M1 == M2 ? 384 : 128) ? 3 : 0;
+enum class TN { none, t32, t64, lds128, t128 };
+static TN tn_kind(int M1, int M2, long K, const double *A, long lda, const double *B, long ldb, int tri) {
+  const long ld = std::max(lda, ldb);
+  if (param("gemm_f64", 1.0) < 1.0 || M1 <= 0 || M2 <= 0 || K <= 0 || ld >= (1L << 24)) return TN::none;
+  const int most = std::max(M1, M2);
+  // (the direct kernels' 32-bit offsets within a tile bound the column length)
+  if (most <= 32) return TN::t32;
+  if (std::min(M1, M2) <= 64 && ld < (1L << 23)) return TN::t64;
+  const bool half = tri && M1 == M2;
+  if (aligned16(A, lda) && aligned16(B, ldb)) {
+    const long nt1 = (M1 + 127) / 128, nt2 = (M2 + 127) / 128, tiles = half ? nt1 * (nt1 + 1) / 2 : nt1 * nt2;
+    const bool slow = (most > 128 && K < 1024) || (tiles > 144 && K < 6L * most) || (!half && tiles > 576);
+    return slow ? TN::none : TN::lds128;
+  }
+  return ld < (1L << 22) && most <= (half ? 384 : 128) ? TN::t128 : TN::none;
 }
 
 bool gemm_f64_tn(int M1, int M2, long K, double alpha, const double *A, long lda, const double *B,
                  long ldb, double beta, double *C, long ldc, int tri, hipStream_t s) {
-  const int kind = alpha == 0.0 ? 0 : tn_kind(M1, M2, K, A, lda, B, ldb, tri);
-  if (!kind) return false;
+  const TN kind = alpha == 0.0 ? TN::none : tn_kind(M1, M2, K, A, lda, B, ldb, tri);
+  if (kind == TN::none) return false;
   Timed t("gemm_f64", 2.0 * (double)M1 * M2 * K);
   TNArgs a{};
   a.A = A; a.B = B; a.lda = lda; a.ldb = ldb; a.K = K; a.M1 = M1; a.M2 = M2;
   a.tri = M1 == M2 ? tri : 0;
-  if (kind == 1) tn_launch<2>(a, false, alpha, beta, C, ldc, s);
-  else tn_launch<4>(a, kind == 2, alpha, beta, C, ldc, s);
+  if (kind == TN::t32) tn_launch<1>(a, false, alpha, beta, C, ldc, s);
+  else if (kind == TN::t64) tn_launch<2>(a, false, alpha, beta, C, ldc, s);
+  else tn_launch<4>(a, kind == TN::lds128, alpha, beta, C, ldc, s);
   return true;
 }
 

@@ -35,6 +35,34 @@ def test_tn_product(kk, m1, m2, k, beta):
     assert np.all(np.abs(C - ref) <= bound)
 
 
+# at most 32 columns (32 x 32 tiles), and either side of the shortest K of the 128 x 128 tiles
+@pytest.mark.parametrize("m1,m2,k", [(2, 32, 1), (32, 32, 4099), (17, 31, 100), (1, 32, 300), (32, 33, 258),
+                                     (200, 131, 1022), (200, 131, 1024)])
+def test_tn_product_narrow(kk, m1, m2, k):
+    test_tn_product(kk, m1, m2, k, -0.5)
+
+
+@pytest.mark.parametrize("m,ld", [(32, 16_700_000), (64, 8_380_000), (64, 8_388_610)])
+def test_tn_product_long_columns(kk, m, ld):
+    """Columns so far apart that the last one of a tile lies almost 2^32 bytes from the first (the
+    direct kernels' offsets), and one length past that for 64 columns; bound as above."""
+    k = 70
+    rng = np.random.default_rng(m)
+    dev, host = [], []
+    for _ in range(2):
+        x = rng.standard_normal((m, k))
+        d = kk.DeviceArray((ld, m))
+        for j in range(m):
+            kk._ck(kk.lib().kukan_memcpy(d.device_ptr + 8 * ld * j, x[j].ctypes.data, 8 * k, 1), "kukan_memcpy")
+        kk.synchronize()
+        dev.append(d)
+        host.append(x)
+    C = np.full((m, m), np.nan, order="F")
+    kk.subspace_gemm(1, m, m, k, 0.7, dev[0], ld, dev[1], ld, 0.0, C, m)
+    ref = 0.7 * (host[0].astype(np.longdouble) @ host[1].astype(np.longdouble).T)
+    assert np.all(np.abs(C - ref) <= (k + 4) * 2.0 ** -53 * 0.7 * (np.abs(host[0]) @ np.abs(host[1]).T))
+
+
 @pytest.mark.parametrize("n,m", [(12, 5), (11, 70), (12, 129), (16, 300)])
 def test_orthogonalisation_triangles(kk, n, m):
     """orthogonalization_r forms a Gram triangle and applies the triangular inverse in place, over
