@@ -462,7 +462,8 @@ static unsigned nn_grid(const NNArgs64 &a) { return (unsigned)((a.row_blocks + 7
 bool gemm_f64_nn_upper(long R, int K, int M2, double alpha, const double *X, long ldx, const double *C, long ldc,
                        double beta, double *Y, long ldy, hipStream_t s) {
   if (M2 <= 64 || alpha == 0.0 || !nn_ok(X, ldx, Y, ldy, R, K, M2)) return false;
-  Timed t("gemm_f64", 2.0 * (double)R * M2 * K);
+  const double k = std::min(K, M2);  // column j takes its first j + 1 rows, at most K
+  Timed t("gemm_f64", (double)R * (k * (k + 1.0) + 2.0 * K * (M2 - k)));
   NNArgs64 a = nn_prepare(R, K, M2, alpha, X, ldx, C, ldc, Y, ldy, s);
   a.beta = beta;
   hipLaunchKernelGGL(k_nn_f64, dim3(nn_grid(a)), dim3(256), 0, s, a);
@@ -523,7 +524,8 @@ bool gemm_f64_tn(int M1, int M2, long K, double alpha, const double *A, long lda
                  long ldb, double beta, double *C, long ldc, int tri, hipStream_t s) {
   const TN kind = alpha == 0.0 ? TN::none : tn_kind(M1, M2, K, A, lda, B, ldb, tri);
   if (kind == TN::none) return false;
-  Timed t("gemm_f64", 2.0 * (double)M1 * M2 * K);
+  // the flops of the entries asked for: of a triangle M1 (M1 + 1) / 2
+  Timed t("gemm_f64", (double)K * M1 * (tri && M1 == M2 ? M1 + 1.0 : 2.0 * M2));
   TNArgs a{};
   a.A = A; a.B = B; a.lda = lda; a.ldb = ldb; a.K = K; a.M1 = M1; a.M2 = M2;
   a.tri = M1 == M2 ? tri : 0;

@@ -120,3 +120,31 @@ def test_block_cg_projection_triangle(kk, m):
     np.testing.assert_allclose(out[0]["sval"], out[1]["sval"], rtol=0, atol=1e-10 * np.abs(out[1]["sval"]).max())
     rho = [(o["svecre"] ** 2).sum(axis=1) for o in out]
     np.testing.assert_allclose(rho[0], rho[1], rtol=0, atol=1e-9 * rho[1].max())
+
+
+def test_timed_flops(kk):
+    """The work booked beside a product's time: 2 m1 m2 k of a full one, half of it (with the
+    diagonal) where one triangle is asked for."""
+    m, n = 200, 16
+    s = synth.make_system(n, 0.4, 2, m, seed=1)
+    psi = synth.random_bands(s)
+    st = dict(svecre=psi, ssvre=psi, rspsep=np.zeros((9, s.natom, m), order="F"))
+
+    def booked(f):
+        kk.timing_reset()
+        kk.set_param("timing", 1)
+        f()
+        kk.synchronize()
+        kk.set_param("timing", 0)
+        return kk.timing()["gemm_f64"][2]
+    C = np.zeros((m, m), order="F")
+    assert booked(lambda: kk.subspace_gemm(1, m, m, s.npts, 1.0, psi, s.npts, psi, s.npts, 0.0, C, m)) == 2 * m * m * s.npts
+    gram = booked(lambda: kk.call("orthogonalization_r", **synth.abi_args(s), nflag=1, **st))
+    assert gram == m * (m + 1) * s.npts
+    # one block-CG step: the Gram triangles before and after, the projection's two
+    kw = dict(synth.abi_args(s, nsdmax=1, epssd=1e-14), hsvre=np.zeros_like(psi, order="F"), sval=np.zeros(m),
+              residual_states=np.zeros(m))
+    kk.set_param("kscg_mode", 1)
+    total = booked(lambda: kk.call("kscg_r", **kw, **st))
+    kk.set_param("kscg_mode", 0)
+    assert total == 4 * gram
