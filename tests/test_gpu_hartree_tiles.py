@@ -58,6 +58,14 @@ def test_tiles(kk, dims, nperi, nfh):
     assert kk.get_param("hartree_iterations") < 3000
 
 
+# 1064 and 1300 tiles of 32 x 8 / 16 x 16 columns by four planes (four from 1024 tiles on), 8320 and
+# 8280 (eight past 8192), every edge ending inside a tile
+@pytest.mark.parametrize("dims,nperi,nfh", [((124, 56, 149), 3, 4), ((124, 55, 150), 0, 6), ((70, 66, 205), 1, 5),
+                                            ((250, 121, 257), 3, 6), ((251, 122, 259), 1, 4), ((248, 119, 273), 2, 5)])
+def test_taller_tiles(kk, dims, nperi, nfh):
+    test_tiles(kk, dims, nperi, nfh)
+
+
 def test_lock_step(kk):
     """Cells of different edges advanced together, their rule changed from step to step (an
     iteration count inside, at and past a block of 16): each against its own solve from the same
@@ -73,6 +81,33 @@ def test_lock_step(kk):
         cells.append([s, np.zeros(s.npts)])
     z = np.zeros(1)
     for batched, ncgmax in ((True, 1), (True, 16), (False, 17), (True, 33), (False, 1), (True, 15)):
+        b.step(batched=batched, ncgmax=ncgmax, epsvh=1e-30)
+        for i, (s, start) in enumerate(cells):
+            psi, _, vh, its = b.get(i)
+            ref = start.copy()
+            kk.call("scf_hartree", nd=1, ncpx_d=s.n, ncpy_d=s.n, ncpz_d=s.n, nfh=4, ndisp=6, nperi=3, ncgres=801,
+                    ncgmin=1, ncgmax=ncgmax, xmax=s.xmax, ymax=s.xmax, zmax=s.xmax, epsvh=1e-30,
+                    rho_aug_dense=(psi ** 2).sum(axis=1), boundx=z, boundy=z, boundz=z, vh_dense=ref)
+            assert its == ncgmax
+            np.testing.assert_allclose(vh, ref, rtol=0, atol=1e-11 * np.abs(ref).max())
+            cells[i][1] = vh.copy()
+    b.close()
+
+
+@pytest.mark.parametrize("sizes", [(66, 70, 62), (150, 149, 131)])
+def test_lock_step_taller_tiles(kk, sizes):
+    """Cells together large enough for tiles of four and of eight planes (1131 tiles of 16 x 16
+    columns by four planes, 10025 of 32 x 8), none of whose edges ends with a tile; bar as above."""
+    from rspacedist_amd import batch, synth
+    b = batch.Batch()
+    cells = []
+    for n in sizes:
+        s = synth.make_system(n, 0.3, 1, 1, seed=n)
+        psi = np.asfortranarray(synth.random_bands(s))
+        b.add(s, psi / np.linalg.norm(psi) / np.sqrt(s.dv))
+        cells.append([s, np.zeros(s.npts)])
+    z = np.zeros(1)
+    for batched, ncgmax in ((True, 5), (False, 18)):
         b.step(batched=batched, ncgmax=ncgmax, epsvh=1e-30)
         for i, (s, start) in enumerate(cells):
             psi, _, vh, its = b.get(i)

@@ -65,3 +65,39 @@ def test_iterates(kk, orc, case, cplx):
     np.testing.assert_allclose(g["residual_states"], o["residual_states"], rtol=1e-6, atol=1e-14)
     assert g["_ret"]["ksitmax"] == o["_ret"]["ksitmax"]
     assert g["_ret"]["ksconv"] == o["_ret"]["ksconv"]
+
+
+@pytest.mark.parametrize("cplx", [False, True])
+@pytest.mark.parametrize("dims,nf", [((17, 17, 260), 4), ((17, 18, 1030), 3), ((18, 17, 1029), 8)])
+def test_long_grids(kk, orc, dims, nf, cplx):
+    """More tiles than the H kernel's 512 work-groups (520 tiles of two planes), and enough for
+    tiles of four planes (past 2048 of two; a last one of two planes or one), with partial tiles
+    along every axis and vectors longer than one sweep of the elementwise kernels.  Bar as above,
+    for sums over 75000 to 315000 terms."""
+    m, n = 3, int(np.prod(dims))
+    s = synth.make_system(12, 0.45, 3, m, seed=sum(dims), nf=nf, q_scale=1.0)
+    rng = np.random.default_rng(nf)
+    kw = dict(zip(("ncpx", "ncpy", "ncpz"), dims), nperi=3, nsdmax=2, epssd=1e-14,
+              veff=np.asfortranarray(0.3 * rng.standard_normal((n, 1))))
+    psi = rng.standard_normal((n, m))
+    z = lambda *d: np.zeros(d, dtype=np.complex128 if cplx else np.float64, order="F")  # noqa: E731
+    if cplx:
+        psi = psi + 1j * rng.standard_normal((n, m))
+        name, gs, args = "kscg_c", "orthogonalization_c", synth.bloch_args(s, K, **kw)
+        st = dict(sveccm=np.asfortranarray(psi), ssvcm=z(n, m), cspsep=z(9, s.natom, m))
+        vec = ("sveccm", "ssvcm", "hsvcm", "cspsep")
+    else:
+        name, gs, args = "kscg_r", "orthogonalization_r", synth.abi_args(s, **kw)
+        st = dict(svecre=np.asfortranarray(psi), ssvre=z(n, m), rspsep=z(9, s.natom, m))
+        vec = ("svecre", "ssvre", "hsvre", "rspsep")
+    orc.call(gs, **args, nflag=1, **st)
+    st.update({vec[2]: z(n, m), "sval": np.zeros(m), "residual_states": np.zeros(m)})
+    out = []
+    for f in (kk.call, orc.call):
+        a = {k: v.copy(order="F") for k, v in st.items()}
+        f(name, **args, **a)
+        out.append(a)
+    g, o = out
+    for k in vec + ("sval",):
+        np.testing.assert_allclose(g[k], o[k], rtol=0, atol=1e-8 * np.abs(o[k]).max(), err_msg=k)
+    np.testing.assert_allclose(g["residual_states"], o["residual_states"], rtol=1e-6, atol=1e-14)
