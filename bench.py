@@ -64,9 +64,9 @@ def run_mode(cell, kk, precision, steps):
 
 
 # timing tag -> kernel whose calibrated HBM bytes per launch the committed counter profile holds
-TRAFFIC_KERNEL = {"gemm_mixed_nn": "k_gemm_nn<3>", "gemm_mixed_tn": "k_gemm_tnf<3>",
-                  "hpsi_stencil": "k_stencil_lds<4, 2, 3>", "hp_comb_stencil": "k_stencil_lds<4, 1, 5>",
-                  "precond_resid": "k_stencil_lds<1, 2, 1>", "update_precond": "k_stencil_lds<1, 1, 6>",
+TRAFFIC_KERNEL = {"gemm_mixed_nn": "k_gemm_nn<3, 4, 5>", "gemm_mixed_tn": "k_gemm_tnf<3>",
+                  "hpsi_stencil": "k_stencil_lds<4, 2, 3, 512>", "hp_comb_stencil": "k_stencil_lds<4, 2, 5, 1024>",
+                  "precond_resid": "k_stencil_lds<1, 2, 1, 512>", "update_precond": "k_stencil_lds<1, 1, 6, 512>",
                   "band_update_dots": "k_pair_update_dots", "p_update_dots": "k_pupdate_dots",
                   "dots": "k_dot_part", "gemm_scale": "k_colmax", "nl_expand": "k_expand_rows<16>",
                   "nl_gather": "k_gather<9, 4>"}
@@ -89,9 +89,9 @@ MFMA_TAGS = {"gemm_f64": PEAK_FP64_TFS, "syrk_f64": PEAK_FP64_TFS, "trsm_f64": P
 
 
 def roofline_entry(tim, tag):
-    """Achieved vs peak for one timing tag from its algorithmic work (HBM bytes, or flops of
-    the full product for the subspace GEMMs: 2 N M^2 whatever triangle or split is computed).
-    For a split-precision product, mfma_pass_frac is the MFMA pipe's share of peak on the
+    """Achieved vs peak for one timing tag from its algorithmic work (HBM bytes, or flops: of
+    the entries asked for in an FP64 product, of the full product, 2 N M^2 whatever triangle or split
+    is computed, in a split-precision one).  For the latter, mfma_pass_frac is the MFMA pipe's share of peak on the
     f16 flops it actually issued (three passes per product over the tiles computed)."""
     ms, cnt, work = tim.get(tag, (0.0, 0, 0.0))
     if cnt == 0 or ms == 0:
@@ -240,7 +240,8 @@ def config3(kk):
     kern = {k: v for k, v in tim.items() if not k.startswith("phase_") and v[1] > 0}
     return {"workload": "96^3 h=0.2, 256 bands, 32 atoms: E = sum <psi|H|psi> + E_H and dE/dV_loc, dE/dR by torch.autograd",
             "forward_s": round(t1 - t0, 4), "backward_s": round(t2 - t1, 4), "energy_Ha": float(E),
-            "kernels": {k: roofline_entry(tim, k) for k in kern if kern[k][2] > 0}}
+            # the committed counters are of the 128^3 step's launches
+            "kernels": {k: dict(roofline_entry(tim, k), traffic=None) for k in kern if kern[k][2] > 0}}
 
 
 def config4(kk):

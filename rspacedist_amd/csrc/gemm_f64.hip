@@ -490,9 +490,10 @@ void gemm_f64_apply_upper(long R, int M, double *X, long ldx, const double *C, l
 
 // Which TN kernel, from times at K = 512 .. 8000000 (rocBLAS dgemm beside them; its times jump between
 // neighbouring sizes, and many are ten times these):
-//  - at most 32 columns on both sides: 32 x 32 tiles;
+//  - at most 32 columns on both sides: 32 x 32 tiles (4096000 x 16 0.34 ms, in 64 x 64 tiles, whose
+//    padding is multiplied too, 0.56, dgemm 0.37; 64000 x 32 0.028, 0.034 and 10.2);
 //  - at most 64 on one side: 64 x 64 tiles.  rocBLAS runs the whole K in one tile's work-group
-//    there: 64000 x 32 takes 10.3 ms against 0.034 ms, 884736 x 64 1.70 against 0.27;
+//    there: 64000 x 64 takes 10.2 ms against 0.036 ms, 884736 x 64 1.70 against 0.26;
 //  - 16-byte aligned columns: 128 x 128 tiles through LDS, 73-75 TFLOP/s from 384 columns on
 //    (884736 x 512: 6.34 ms against 8.0; its triangle 4.23 against 5.9 in 256-column blocks;
 //    2097152 x 1024, the triangle: 33.7 against 44.5).  Past 128 columns a short K does not repay

@@ -412,7 +412,7 @@ __global__ __launch_bounds__(64) void k_force_sum(const int *act, const int *is_
   if (threadIdx.x == 0) fa[(long)d * natom + act[5 * ia + 3]] -= 2.0 * s;
 }
 
-// rho(:,s) (=|+=) scale sum_l f_l psi_l^2 over all bands, band order (scf_charge8f.F90:303-318):
+// rho(:,s) = scale ([rho +] sum_l f_l psi_l^2) over all bands, band order (scf_charge8f.F90:303-318):
 // one launch, eight bands' loads in flight per point (with one launch per 64 bands rho was
 // cleared, read and written between them; 40^3 x 32: 26 -> 18 us for the call)
 __global__ __launch_bounds__(256) void k_charge(long n, int nb, const double *psi, long ld, const double *f,
@@ -1817,7 +1817,8 @@ int hartree(const HartreeArgs &a, const HartreeWork *ws) {
   int *state = B.state;
   const double dvo = g.dv() / omega;
   lib().params["hartree_persistent_used"] = 0.0;
-  // opt-in: one cooperative launch (47 us per iteration at 128^3, 45 / 38 at 96^3 / 64^3)
+  // opt-in: one cooperative launch (47 us per iteration at 128^3, 45 / 38 at 96^3 / 64^3; the launch
+  // pairs below take 38, 24 and 16)
   if (!ws && param("hartree_persistent", 0.0) >= 1.0) {
     HIPCK(hipMemcpyAsync(B.p2, ap, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
     HIPCK(hipMemcpyAsync(p, r, sizeof(double) * n, hipMemcpyDeviceToDevice, s));

@@ -115,7 +115,7 @@ struct HartreeWork {
 // ws: run on the caller's workspace with eager launches (no graph, no allocation)
 int hartree(const HartreeArgs &a, const HartreeWork *ws = nullptr);
 void correct_potential(long n, double dvol_over_omega, double *vh);
-// rho (=|+= with add) scale sum_l f_l psi_l^2
+// rho = scale sum_l f_l psi_l^2, or with add scale (rho + sum_l f_l psi_l^2)
 void charge(long n, int M, const double *psi, const double *f, double *rho, bool add, double scale = 1.0);
 // e_l = dV <psi_l|H|psi_l> (H = T + veff + nonlocal with dij)
 void band_energy(Ctx &c, int M, const double *veff, const double *psi, double *eband);
