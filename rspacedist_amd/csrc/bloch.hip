@@ -131,8 +131,8 @@ __global__ void k_zexpand(const int *nzrows, long nnz, const int *row_ptr, const
     const int slot = ent[e].x, k = ent[e].y, iprj = iprj_slot[slot];
     const zt *c = coef + ldco * b + (size_t)nprjmx * slot;
     const double *p = vnl + (size_t)k + (size_t)num_list * (size_t)nprjmx * slot;
-    zt av = zsc(p[0], c[0]);
-    for (int j = 1; j < iprj; j++) av = zadd(av, zsc(p[(size_t)num_list * j], c[j]));
+    zt av = zmk(0.0, 0.0);  // (nothing from an atom whose species has no projectors)
+    for (int j = 0; j < iprj; j++) av = zadd(av, zsc(p[(size_t)num_list * j], c[j]));
     s = zadd(s, zmul(zcj(ph[(size_t)k + (size_t)num_list * slot]), av));
   }
   out[ldo * b + r] = s;

@@ -297,3 +297,38 @@ def test_scf_diag_bloch_diis_converges_to_dense_eigenpairs(kk, orc, q):
     np.testing.assert_allclose(st["sval"], w, rtol=0, atol=1e-7)
     Q = st["sveccm"]
     np.testing.assert_allclose(np.conj(Q.T) @ Sd @ Q * s.dv, np.eye(6), rtol=0, atol=1e-12)
+
+
+def test_species_without_projectors(kk):
+    """An atom whose species has no projectors adds nothing to H psi or S psi, whatever its columns
+    of the table hold and whatever an earlier call left in the library's buffers: the same results
+    bit for bit with random and with zero columns."""
+    s = synth.make_system(10, 0.5, 3, 6, seed=41, q_scale=2.0)
+    rng = np.random.default_rng(41)
+    two = dict(num_spe=2, sss=np.asfortranarray(np.repeat(s.sss, 2, axis=2)), ntyppp=np.ones(2, dtype=np.int32))
+    psi = synth.random_bands_c(s)
+    out = []
+    for fill in (1.0, 0.0):
+        vnl = s.vnlocp.copy(order="F")
+        vnl[:, :, 1] = fill * rng.standard_normal(vnl.shape[:2])
+
+        def state():
+            st = dict(sveccm=psi.copy(order="F"), ssvcm=np.zeros_like(psi),
+                      cspsep=np.zeros((9, s.natom, s.nbands), dtype=np.complex128, order="F"))
+            kk.call("orthogonalization_c", **kw, nflag=1, **st)
+            return dict(st, hsvcm=np.zeros_like(psi), sval=np.zeros(s.nbands), residual_states=np.zeros(s.nbands))
+        for spe, nprj in (([1, 1, 1], [9, 9]), ([1, 2, 1], [9, 0])):
+            kw = dict(synth.bloch_args(s, K, ndiismax=1, l_hsv=1), **two, vnlocp=vnl,
+                      nprj=np.array(nprj, dtype=np.int32), indspe=np.array(spe, dtype=np.int32))
+            res = [state()]
+            a = state()
+            kk.call("rayleighritz_c", **kw, l_rrb=1, **{k: a[k] for k in ZK + ("sval",)})
+            res.append(a)
+            for name in ("kscg_c", "ksdiis_c"):
+                a = state()
+                kk.call(name, **kw, **a)
+                res.append(a)
+        out.append(res)
+    for x, y in zip(*out):
+        for k in ZK + ("sval", "residual_states"):
+            np.testing.assert_array_equal(x[k], y[k], err_msg=k)
