@@ -1574,6 +1574,7 @@ void launch_precond(const Grid &g, const double *in, long ld_in, bool halo_in, i
 void launch_precond_resid_dot(const Grid &g, const double *h, const double *sp, long ld,
                               const double *eps, double sign, double *out, int nb,
                               double *dot_partial, hipStream_t s, unsigned long long *out_max) {
+  if (!stencil_band_fastest_coef(g, false)) throw Error(1, "fused residual preconditioner: the tiled path only");
   Timed t("precond_resid", 8.0 * (double)g.n() * nb * 3.0);
   SL q{};
   q.nx = g.nx; q.ny = g.ny; q.nz = g.nz;

@@ -1349,8 +1349,10 @@ void kscg_block(Ctx &c, const KscgArgs &a, bool ortho_first, bool keep_h) {
   // S = 1: fuse the direction update with its dot products and the band update with the next
   // iteration's <psi|psi> and <psi|H psi> (same arithmetic, fewer passes over HBM)
   const bool fused = c.q_zero;
-  // the combination stencil (H p = fac H P + mdf H psi, p never stored) needs the tiled path
-  const bool comb = fused && stencil_band_fastest_coef(c.g, false) && param("bcg_comb", 1.0) >= 1.0;
+  // the combination stencil (H p = fac H P + mdf H psi, p never stored) and the residual
+  // preconditioner with its dot products need the tiled path (8 points an axis, x at most 256)
+  const bool tiled = stencil_band_fastest_coef(c.g, false);
+  const bool comb = fused && tiled && param("bcg_comb", 1.0) >= 1.0;
   double *eh_next = c.buf("bcg.eh", (size_t)M);
   int *active = (int *)scratch("bcg.active", sizeof(int) * M);
   std::vector<int> act_h(M, 1);
@@ -1397,9 +1399,13 @@ void kscg_block(Ctx &c, const KscgArgs &a, bool ortho_first, bool keep_h) {
     // K r with r = -(H psi - eps S psi), and <r|Kr> (unprojected): residual measure and CG ratio;
     // for split-precision products also the per-band max |K r|
     const bool mixed = mixed_for(n);
-    unsigned long long *krmax = mixed ? (unsigned long long *)c.buf("bcg.krmax", M) : nullptr;
+    unsigned long long *krmax = mixed && tiled ? (unsigned long long *)c.buf("bcg.krmax", M) : nullptr;
     if (kr_ready) {
       HIPCK(hipMemcpyAsync(rnew, rnext, sizeof(double) * M, hipMemcpyDeviceToDevice, c.s));
+    } else if (!tiled) {
+      double *R = c.buf("bcg.R", (size_t)n * M);
+      launch_precond_resid(c.g, hpsi, spsi, n, a.sval, -1.0, R, KR, M, c.s);
+      c.dots(R, n, KR, n, M, rnew);
     } else {
       const int np = stencil_nparts(c.g, 1, M);
       double *part = c.buf("bcg.kpart", (size_t)np * M);
@@ -1414,7 +1420,8 @@ void kscg_block(Ctx &c, const KscgArgs &a, bool ortho_first, bool keep_h) {
     const SplitBands *pre = nullptr;
     if (mixed) {
       double *sk = c.buf("bcg.skr", M);
-      maxscale(krmax, M, sk, c.s);
+      if (krmax) maxscale(krmax, M, sk, c.s);
+      else colscale(KR, n, n, M, sk, c.s);
       s_kr = sk;
       // S = 1: S psi equals psi, so one split of psi serves both products
       if (c.q_zero) pre = split_psi(c, "bcg.psi", psi, M, fused ? gg : nullptr, spl);
